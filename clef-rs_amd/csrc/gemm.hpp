@@ -20,10 +20,9 @@ struct GemmParams {
 // epilogue: 0 store, 1 residual add into f32 y, 2 SwiGLU
 int gemm_launch(const GemmParams& p, int epilogue, hipStream_t stream);
 
-// f16 large-M path (gemm_f16.hip)
+// f16 operands with whole 64-deep K stages and 16-byte rows (gemm_f16.hip)
 bool gemm_f16_dma_ok(const GemmParams& p);
 int gemm_f16_dma_launch(const GemmParams& p, int epilogue, hipStream_t stream);
-int gemm_f16_tile_shape(const GemmParams& p, int epilogue, int* bm);  // width 256, 192 or 128; rows 256 or 128
 
 // a/b projections fused with the DeltaNet gates (gemm_f16.hip); f16 operands,
 // Hv in {16, 32, 64}, K % 256 == 0, K <= 4096, rows 16-byte aligned (checked

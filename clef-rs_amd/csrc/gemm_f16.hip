@@ -1,7 +1,8 @@
-// f16 projection GEMM for large row counts: y = x . W^T, x [M,K], W [N,K]
+// f16 projection GEMM: y = x . W^T, x [M,K], W [N,K]
 // (both K-contiguous), f32 accumulation.  Same contract and epilogues as
 // gemm.hip (neural.metal:7-125 tile GEMM, projection.rs:82-95); selected for
-// M >= 256, K % 64 == 0 and 16-byte aligned rows.
+// K % 64 == 0 and 16-byte aligned rows.  Launches that these tiles would
+// leave mostly idle take gemm_ring.hpp's smaller ones.
 //
 // A work-group of 8 waves (4 x 2, two per SIMD) computes a 256 x BN tile
 // (or 128 x BN when 256-row tiles would leave CUs idle), each wave
@@ -33,11 +34,12 @@
 
 #include "common.hpp"
 #include "gemm.hpp"
+#include "gemm_dma.hpp"
+#include "gemm_ring.hpp"
 
 namespace clef {
 
-// CUs of the current device (cached per device)
-static int device_cus() {
+int device_cus() {
   static int cached[64] = {0};
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
@@ -51,41 +53,7 @@ static int device_cus() {
 
 namespace {
 
-constexpr int kBM = 256, kBK = 64;  // largest row tile, K stage
-
-// buffer_load_dwordx4 ... lds written as inline asm: the compiler does not
-// see an LDS write it would have to order before every later LDS read (it
-// would wait for all DMAs in flight, i.e. for the next stage, before
-// computing on the current one).  Completion is awaited explicitly (vmcnt)
-// before the barrier that publishes a stage.  The source is a buffer resource
-// (SGPR base and size) plus a 32-bit lane byte offset; the LDS destination
-// goes in M0 (low 32 bits of the LDS address), lane l writing 16 bytes at
-// M0 + 16 l.  The asm carries the one wait state an LDS DMA needs after the
-// SALU write of M0.  (1-6% faster than global_load_lds_dwordx4 with 64-bit
-// lane addresses on the projection shapes, bit-identical.)
-__device__ __forceinline__ void bdma16(__amdgpu_buffer_rsrc_t r, uint32_t off, void* lds_block) {
-  const uint32_t m0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds_block));
-  asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(r), "{m0}"(m0) : "memory");
-}
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t operand_rsrc(const half_t* base, int64_t rows, int64_t ld) {
-  // rows * ld * 2 < 2^32 (checked by gemm_f16_dma_ok)
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(base), 0, static_cast<int>(static_cast<uint32_t>(rows * ld * 2)),
-                                           0x00020000);
-}
-
-__device__ __forceinline__ void vm_wait_all() { __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8)); }
-template <int N>
-__device__ __forceinline__ void vm_wait() {  // s_waitcnt vmcnt(N)
-  static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
-}
-// vmcnt(n) for an n that is a constant once loops are unrolled
-template <int... Ns>
-__device__ __forceinline__ void vm_wait_n(int n, std::integer_sequence<int, Ns...>) {
-  ((n == Ns ? (vm_wait<Ns>(), 0) : 0), ...);
-}
-__device__ __forceinline__ void vm_wait_n(int n) { vm_wait_n(n, std::make_integer_sequence<int, 40>{}); }
-
+constexpr int kBK = 64;  // K stage
 
 template <int BM, int BN, int VM, int NSA, int NSB, int EPI, bool PERSIST>
 __global__ __launch_bounds__(VM * 128) void gemm_f16_dma(GemmParams p) {
@@ -1109,43 +1077,86 @@ int ab_gates_f16_launch(const void* x, int64_t ldx, const void* packed, int K, c
 // (the DMA reads x and the weights through buffer resources: byte offsets
 // below 2^32)
 bool gemm_f16_dma_ok(const GemmParams& p) {
-  return p.dtype_in == 1 && p.vec && p.M >= kBM && p.K % kBK == 0 &&
-         (int64_t)p.M * p.ldx < (int64_t(1) << 31) && (int64_t)p.N * p.ldw < (int64_t(1) << 31);
+  return p.dtype_in == 1 && p.vec && p.K % kBK == 0 && (int64_t)p.M * p.ldx < (int64_t(1) << 31) &&
+         (int64_t)p.N * p.ldw < (int64_t(1) << 31);
 }
 
-
-// Tile shape: one tile per CU at a time (the LDS holds one), so a launch
-// takes ceil(tiles / CUs) rounds, each as long as a tile; a smaller tile
-// costs a little more per output (fewer products per fragment read and per
-// byte moved).  The shape with the least rounds x area x that cost wins,
-// e.g. 256 x 256 for N = 12288, 256 x 192 for N = 9216 (768 tiles: 3 full
-// rounds instead of 2.25), 256 x 128 for M = 4096, N = 2048 (256 tiles: one
-// round), 128 x 128 for M = N = 2048 (256 tiles instead of 128 of 256 x 128,
-// which leave half the CUs idle).  SwiGLU keeps widths 256 or 128 (its wave
-// columns pair gate and up blocks).  Returns the width; *bm the row tile.
-int gemm_f16_tile_shape(const GemmParams& p, int epilogue, int* bm) {
+// Tile shape.  The large tiles hold one work-group per CU, so a launch takes
+// ceil(tiles / CUs) rounds, each as long as a tile; a smaller tile costs a
+// little more per output (fewer products per fragment read and per byte
+// moved).  The shape with the least rounds x area x that cost wins, e.g.
+// 256 x 256 for N = 12288, 256 x 192 for N = 9216 (768 tiles: 3 full rounds
+// instead of 2.25), 256 x 128 for M = 4096, N = 2048 (256 tiles: one round),
+// 128 x 128 for M = N = 2048 (256 tiles instead of 128 of 256 x 128, which
+// leave half the CUs idle).  SwiGLU keeps widths 256 or 128 (its wave columns
+// pair gate and up blocks).
+//
+// The ring kernel's small tiles (gemm_ring.hpp) enter with their measured
+// time of a round in the same unit (1400 per us at K = 2048: 128 x 128 takes
+// 17.5 us, 64 x 64 10); two work-groups of a 32 x 16 or 64 x 32 tile share a
+// CU, and each further round adds half of the first's time.  Where the lines
+// fall for N = 2048, K = 6144 (us, before -> now; weights from HBM): M = 33
+// on 32 x 16 109 -> 12.6, M = 200 on 64 x 32 120 -> 22.6, M = 500 on 64 x 64
+// 57.7 -> 31.7, M = 1000 on 128 x 64 56.6 -> 44.9, M = 1500 stays on
+// 128 x 128 (57.8; 128 x 64 76.5).  N = 12288, K = 2048: M = 33 on 64 x 64
+// 39.5 -> 13.1, M = 100 on 128 x 64 40.8 -> 16.9, M = 300 stays on 128 x 128
+// (28.9; 64 x 64 38.1).
+enum RingTile { kRingNone, kRing32x16, kRing64x32, kRing64x64, kRing128x64 };
+struct TileShape {
+  int bm, bn;
+  RingTile ring;
+};
+static TileShape gemm_f16_tile_shape(const GemmParams& p, int epilogue) {
   const int n_eff = epilogue == 2 ? 2 * p.N : p.N;
   const long cus = device_cus();
-  auto cost = [&](int rows, int bn, double per_out) {
+  auto rounds = [&](int rows, int bn) {
     const long tiles = (long)((p.M + rows - 1) / rows) * ((n_eff + bn - 1) / bn);
-    return (double)((tiles + cus - 1) / cus) * rows * bn * per_out;
+    return (double)((tiles + cus - 1) / cus);
   };
-  struct Cand { int bm, bn; double c; };
-  const Cand cands[] = {{256, 256, cost(256, 256, 1.0)},
-                        {256, 192, epilogue == 2 ? 1e300 : cost(256, 192, 1.1)},
-                        {256, 128, cost(256, 128, 1.2)},
-                        {128, 128, cost(128, 128, 1.5)}};
+  auto cost = [&](int rows, int bn, double per_out) { return rounds(rows, bn) * rows * bn * per_out; };
+  auto paired = [&](int rows, int bn, double unit) { return (0.5 + 0.5 * rounds(rows, bn)) * unit; };
+  struct Cand {
+    TileShape t;
+    double c;
+  };
+  const Cand cands[] = {{{256, 256, kRingNone}, cost(256, 256, 1.0)},
+                        {{256, 192, kRingNone}, epilogue == 2 ? 1e300 : cost(256, 192, 1.1)},
+                        {{256, 128, kRingNone}, cost(256, 128, 1.2)},
+                        {{128, 128, kRingNone}, cost(128, 128, 1.5)},
+                        {{128, 64, kRing128x64}, rounds(128, 64) * 20000.0},
+                        {{64, 64, kRing64x64}, rounds(64, 64) * 14000.0},
+                        {{64, 32, kRing64x32}, paired(64, 32, 10200.0)},
+                        {{32, 16, kRing32x16}, epilogue == 2 ? 1e300 : paired(32, 16, 5900.0)}};
   Cand best = cands[0];
   for (const Cand& c : cands)
     if (c.c < best.c) best = c;
-  *bm = best.bm;
-  return best.bn;
+  return best.t;
+}
+
+template <int BM, int BN, int VM, int VN, int U, int S>
+static int launch_ring(const GemmParams& p, int epilogue, hipStream_t s) {
+  const int on = epilogue == 2 ? BN / 2 : BN;
+  const dim3 grid((unsigned)(((p.M + BM - 1) / BM) * ((p.N + on - 1) / on)));
+  if (epilogue == 0)
+    hipLaunchKernelGGL((gemm_f16_ring<BM, BN, VM, VN, U, S, 0>), grid, dim3(512), 0, s, p);
+  else if (epilogue == 1)
+    hipLaunchKernelGGL((gemm_f16_ring<BM, BN, VM, VN, U, S, 1>), grid, dim3(512), 0, s, p);
+  else if constexpr (BN >= 32)  // a SwiGLU wave holds gate and up columns of its outputs: 32 or more
+    hipLaunchKernelGGL((gemm_f16_ring<BM, BN, VM, (BN / VN >= 32 ? VN : BN / 32), U, S, 2>), grid, dim3(512), 0, s, p);
+  return check_launch("gemm");
 }
 
 int gemm_f16_dma_launch(const GemmParams& p, int epilogue, hipStream_t s) {
-  int bm = kBM;
-  const int bn = gemm_f16_tile_shape(p, epilogue, &bm);
-  if (bm == 128) {
+  const TileShape t = gemm_f16_tile_shape(p, epilogue);
+  const int bn = t.bn;
+  switch (t.ring) {
+    case kRing32x16: return launch_ring<32, 16, 2, 1, 4, 3>(p, epilogue, s);
+    case kRing64x32: return launch_ring<64, 32, 4, 2, 2, 3>(p, epilogue, s);
+    case kRing64x64: return launch_ring<64, 64, 4, 2, 2, 5>(p, epilogue, s);
+    case kRing128x64: return launch_ring<128, 64, 4, 2, 2, 3>(p, epilogue, s);
+    case kRingNone: break;
+  }
+  if (t.bm == 128) {
     if (epilogue == 0) return launch<128, 128, 0>(p, s);
     if (epilogue == 1) return launch<128, 128, 1>(p, s);
     return launch<128, 128, 2>(p, s);

@@ -218,3 +218,45 @@ def test_silu_mul_rejects_bad_arguments(clef):
     assert clef.lib().clef_silu_mul(None, None, None, 16, 1, None) < 0
     assert clef.lib().clef_silu_mul(1, 1, 1, 0, 1, None) < 0
     assert clef.lib().clef_silu_mul(1, 1, 1, 16, 7, None) < 0
+
+
+# launches on small tiles (32 x 16, 64 x 32, 64 x 64, 128 x 64): one row, tile
+# edges and remainders in rows and columns, odd row pitches, one K stage,
+# partial stages (K = 320, 192), a request-sized call of each projection
+SMALL = [(1, 2048, 6144), (33, 2048, 6144), (31, 100, 64), (64, 1000, 320), (65, 73, 192), (200, 2048, 4096),
+         (129, 2047, 1024), (1, 12288, 2048), (37, 12288, 2048), (100, 12288, 2048), (300, 2048, 2048),
+         (500, 2000, 512), (1000, 2048, 6144)]
+
+
+@gpu
+@pytest.mark.parametrize("M,N,K", SMALL)
+def test_gemm_small_tiles(clef, M, N, K):
+    """Each epilogue against the reference, and equal bit for bit to the same
+    rows of a call with enough rows for the large tiles (one summation order)."""
+    x, w = _inputs(21, M, N, K, torch.float16)
+    _, u = _inputs(22, 1, N, K, torch.float16)
+    rows = 4096 * 3
+    xl = torch.cat([x, torch.zeros((rows - M, K), dtype=x.dtype, device="cuda")])
+    y = clef.gemm(x, w)
+    _check_f16(y, x, w)
+    assert torch.equal(y, clef.gemm(xl, w)[:M])
+    assert torch.equal(clef.gemm(x, w, out_dtype=torch.float32).half(), y)
+    h0 = torch.randn((M, N), device="cuda")
+    h = clef.gemm(x, w, residual=h0.clone(), out_dtype=torch.float16)
+    assert torch.equal(h, h0 + y.float())
+    s = clef.gemm_swiglu(x, w, u)
+    assert torch.equal(s, clef.silu_mul(y, clef.gemm(x, u)))
+    assert torch.equal(s, clef.gemm_swiglu(xl, w, u)[:M])
+
+
+@gpu
+def test_gemm_small_tiles_write_only_their_rows(clef):
+    """Strided operands and outputs (views into wider buffers): nothing outside
+    the output's rows and columns is written."""
+    M, N, K = 45, 90, 128
+    xb, wb = _inputs(23, M, N, 2 * K, torch.float16)
+    x, w = xb[:, K:], wb[:, :K]
+    buf = torch.full((M + 3, N + 30), 7.0, device="cuda").half()
+    clef.gemm(x, w, out=buf[:M, 8:8 + N])
+    _check_f16(buf[:M, 8:8 + N], x, w)
+    assert (buf[M:] == 7).all() and (buf[:, :8] == 7).all() and (buf[:, 8 + N:] == 7).all()
