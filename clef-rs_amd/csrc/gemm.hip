@@ -1,4 +1,6 @@
 // Projection GEMMs y = x . W^T for gfx950 (x [M,K], W [N,K], both K-contiguous).
+// The general kernel: any K and alignment; f16 operands with whole 64-deep
+// stages run in gemm_f16.hip, f32 operands with 16-byte rows in gemm_f32.hpp.
 //
 // Replaces the reference's tile GEMM (crates/core/src/models/neural.metal:7-125,
 // dispatch neural.rs:201-280) and candle_nn::Linear (projection.rs:82-95).
@@ -14,16 +16,15 @@
 //
 // f32 operands: each BK = 32 stage is accumulated in a fresh accumulator and
 // then added to the running sum, which cuts the rounding error of a K = 6144
-// dot product roughly fourfold against one accumulator chain over all of K
-// (that is what keeps the f32 profile within 1e-5 of an exactly accumulated
-// product at the block shape); the second accumulator set caps f32 tiles at
-// 256 x 128.
+// dot product roughly fourfold against one accumulator chain over all of K;
+// the second accumulator set caps f32 tiles at 256 x 128.
 //
 // Epilogues: store (f16 rounded once from the f32 accumulator, or f32);
 // residual (h += to_f32(round(acc)), the residual add of qwen.rs:399-410);
 // SwiGLU (silu(gate) * up with the half roundings of neural.metal:29-44).
 #include "common.hpp"
 #include "gemm.hpp"
+#include "gemm_f32.hpp"
 
 namespace clef {
 namespace {
@@ -291,8 +292,49 @@ int launch_epi(const GemmParams& p, hipStream_t s) {
 
 }  // namespace
 
+// f32 operands with 16-byte rows: the bf16 split kernel (gemm_f32.hpp), whose
+// buffer resources address up to 384 rows by 31-bit byte offsets.
+static bool gemm_f32_split_ok(const GemmParams& p) {
+  return p.dtype_in == 0 && p.vec && p.ldx <= (1 << 20) && p.ldw <= (1 << 20);
+}
+
+template <int BM, int BN, int VM, int VN, int U, int D, bool FAST>
+static int launch_f32_split(const GemmParams& p, int epilogue, hipStream_t s) {
+  const int on = epilogue == 2 ? BN / 2 : BN;
+  const dim3 grid((unsigned)(((p.M + BM - 1) / BM) * ((p.N + on - 1) / on)));
+  if (epilogue == 0)
+    hipLaunchKernelGGL((gemm_f32_split<BM, BN, VM, VN, U, D, FAST, 0>), grid, dim3(512), 0, s, p);
+  else if (epilogue == 1)
+    hipLaunchKernelGGL((gemm_f32_split<BM, BN, VM, VN, U, D, FAST, 1>), grid, dim3(512), 0, s, p);
+  else  // a SwiGLU wave holds gate and up columns of its outputs: 32 or more
+    hipLaunchKernelGGL((gemm_f32_split<BM, BN, VM, (BN / VN >= 32 ? VN : BN / 32), U, D, FAST, 2>), grid, dim3(512), 0,
+                       s, p);
+  return check_launch("gemm");
+}
+
+// Tile with the least rounds of 256 work-groups x time of a round (us at K =
+// 2048, weights from HBM; one work-group per CU, and it walks K at the same
+// pace however many there are).  Where the lines fall (us, f32 MFMA kernel ->
+// now): N = 2048, K = 6144: M = 33 on 32 x 32 504 -> 57, M = 500 on 64 x 64
+// 508 -> 141, M = 2048 on 128 x 128 512 -> 325; N = 12288, K = 2048: M = 33 on
+// 32 x 32 or 64 x 64 171 -> 45, M = 200 on 128 x 128 176 -> 104, M = 2048 on
+// 256 x 128 977 -> 552.
+static int gemm_f32_split_launch(const GemmParams& p, int epilogue, hipStream_t s) {
+  const int n_eff = epilogue == 2 ? 2 * p.N : p.N;
+  auto cost = [&](int bm, int bn, double round) {
+    const long tiles = (long)((p.M + bm - 1) / bm) * ((n_eff + bn - 1) / bn);
+    return (double)((tiles + 255) / 256) * round;
+  };
+  const double c256 = cost(256, 128, 165), c128 = cost(128, 128, 100), c64 = cost(64, 64, 41), c32 = cost(32, 32, 19);
+  if (c256 <= c128 && c256 <= c64 && c256 <= c32) return launch_f32_split<256, 128, 2, 4, 1, 1, true>(p, epilogue, s);
+  if (c128 <= c64 && c128 <= c32) return launch_f32_split<128, 128, 2, 4, 1, 1, true>(p, epilogue, s);
+  if (c64 <= c32) return launch_f32_split<64, 64, 2, 2, 2, 2, false>(p, epilogue, s);
+  return launch_f32_split<32, 32, 2, 2, 4, 2, false>(p, epilogue, s);
+}
+
 int gemm_launch(const GemmParams& p, int epilogue, hipStream_t s) {
   if (gemm_f16_dma_ok(p)) return gemm_f16_dma_launch(p, epilogue, s);
+  if (gemm_f32_split_ok(p)) return gemm_f32_split_launch(p, epilogue, s);
   if (p.dtype_in == 1) {
     if (epilogue == 0) return launch_epi<half_t, 0>(p, s);
     if (epilogue == 1) return launch_epi<half_t, 1>(p, s);

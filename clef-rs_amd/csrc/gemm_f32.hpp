@@ -1,0 +1,438 @@
+// f32 projection GEMM on bf16 matrix products (kernel; launched from gemm.hip).
+//
+// An f32 value is the exact sum of three bf16 values (8 + 8 + 8 significant
+// bits, the exponent range of f32), a bf16 product is exact in f32, and
+// v_mfma_f32_16x16x32_bf16 accumulates in f32 at 16 times the rate of the f32
+// MFMA.  x w = sum of nine such products; the six of relative size 2^-18 and
+// above are formed, the dropped three stay below 2^-26 of the term.  Each
+// 32-deep step of K sums its products from zero, small ones first; steps are
+// added up in groups of four and the groups in a running sum, so the sum's
+// own magnitude is rounded once per 128 columns (the f32 MFMA kernel: once per
+// 32, after 16 roundings inside).  Against 64 bits, 2-norm, N(0,1) x N(0,0.02):
+// K = 64 0.58e-7 (f32 MFMA kernel 1.31e-7), K = 320 0.67e-7 (1.20e-7), K =
+// 2048 1.07e-7 (1.79e-7), K = 6144 1.68e-7 (2.74e-7); without the groups 1.60
+// and 2.69e-7 at the last two.
+// Tiles with values that the split does not hold (tiny, infinite, NaN) are
+// formed on the f32 MFMA instead, at the end.
+//
+// The tile's x and weight rows pass through registers (loaded D stages
+// ahead), where they are split, into two LDS buffers of three planes each.
+// What bounds it: at 2048 x 8192 x 2048 (655 -> 363 us) the products run at
+// 1.14 PFLOP/s in bf16, where a large bf16 product of the vendor library
+// reaches 1.29 on this card (the clock drops under random operands); smaller
+// launches by the walk of one work-group along K.  Four tile shapes (launch
+// rule in gemm.hip); all sum in one order, so a row's result does not depend
+// on the shape.  On 256 x 128 and 128 x 128 tiles (FAST) the splitting of the
+// next stage is interleaved with the products of this one, three vector
+// instructions per product: one after the other leaves the matrix cores idle
+// while a wave splits (374 -> 355 us before the groups were added; letting
+// half of the waves multiply first while the others split took 414,
+// single-buffered tiles with two to four work-groups per CU 377 to 420).
+// 256 x 128 as 2 x 4 waves of 128 x 32: as 4 x 2 of 64 x 64 the second set of
+// sums spills (426 us).
+#pragma once
+#include "common.hpp"
+#include "gemm.hpp"
+
+namespace clef {
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float float2_t __attribute__((ext_vector_type(2)));
+typedef uint32_t uint4_t __attribute__((ext_vector_type(4)));
+
+// Stores four consecutive columns c .. c + 3 of row r, clipped to M x N.
+__device__ __forceinline__ void store_row4(const GemmParams& p, int r, int c, const float4_t& o, bool yvec) {
+  if (r >= p.M) return;
+  const int64_t off = (int64_t)r * p.ldy + c;
+  if (p.dtype_out == 1) {
+    const half4 h = {static_cast<half_t>(o[0]), static_cast<half_t>(o[1]), static_cast<half_t>(o[2]),
+                     static_cast<half_t>(o[3])};
+    half_t* dst = static_cast<half_t*>(p.y) + off;
+    if (yvec && c + 3 < p.N) {
+      *reinterpret_cast<half4*>(dst) = h;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (c + e < p.N) dst[e] = h[e];
+    }
+  } else {
+    float* dst = static_cast<float*>(p.y) + off;
+    if (yvec && c + 3 < p.N) {
+      *reinterpret_cast<float4_t*>(dst) = o;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (c + e < p.N) dst[e] = o[e];
+    }
+  }
+}
+
+// x = hi + mid + lo exactly, each a bf16: round to nearest takes 8 bits, and
+// what is left of a 24-bit significand after two of them fits a third.
+__device__ __forceinline__ void split8(const float4_t& a, const float4_t& b, bf16x8& hi, bf16x8& mid, bf16x8& lo) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float2_t x = e < 2 ? float2_t{a[2 * e], a[2 * e + 1]} : float2_t{b[2 * e - 4], b[2 * e - 3]};
+    const bf16x2 h = __builtin_convertvector(x, bf16x2);
+    const float2_t r = x - __builtin_convertvector(h, float2_t);
+    const bf16x2 m = __builtin_convertvector(r, bf16x2);
+    const bf16x2 l = __builtin_convertvector(r - __builtin_convertvector(m, float2_t), bf16x2);
+    hi[2 * e] = h[0], hi[2 * e + 1] = h[1];
+    mid[2 * e] = m[0], mid[2 * e + 1] = m[1];
+    lo[2 * e] = l[0], lo[2 * e + 1] = l[1];
+  }
+}
+
+template <int BM, int BN, int VM, int VN, int U, int D, bool FAST, int EPI>
+__global__ __launch_bounds__(512, 2) void gemm_f32_split(GemmParams p) {
+  constexpr int NT = 512;
+  constexpr int WM = BM / VM, WN = BN / VN, TM = WM / 16, TN = WN / 16;
+  constexpr int ROWS = BM + BN, CPS = ROWS * 4;  // rows and 8-element chunks of a 32-deep sub-stage
+  constexpr int CH = U * CPS / NT;               // chunks per thread per stage
+  constexpr int kPlane = ROWS * 32;              // bf16 of one plane of a sub-stage
+  constexpr int kSub = 3 * kPlane, kBuf = U * kSub;
+  static_assert(VM * VN <= 8 && TM * 16 * VM == BM && TN * 16 * VN == BN, "wave layout");
+  static_assert(U * CPS % NT == 0 && (BM * 4) % 64 == 0, "whole chunks per thread, one operand per wave");
+  static_assert(EPI != 2 || TN % 2 == 0, "a SwiGLU wave holds gate and up columns of the same outputs");
+  static_assert(D == 1 || D == 2, "stages in flight in registers");
+  static_assert(!FAST || (U == 1 && D == 1), "the interleaved loop is one sub-stage deep");
+  static_assert(2 * kBuf * 2 + 16 <= 160 * 1024, "LDS");
+  __shared__ __attribute__((aligned(16))) __bf16 smem[2 * kBuf];
+  __shared__ int tiny_flag;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / VN, wn = wave % VN;
+  constexpr int ON = EPI == 2 ? BN / 2 : BN;  // output columns of a tile
+  // XCD-compact tile order in groups of 4 row tiles, as the f16 kernels'
+  const int tiles_m = (p.M + BM - 1) / BM, tiles_n = (p.N + ON - 1) / ON;
+  const int ntiles = gridDim.x, xcd = blockIdx.x & 7, per = ntiles >> 3, rem = ntiles & 7;
+  const int t = xcd * per + min(xcd, rem) + (blockIdx.x >> 3);
+  const int gsize = 4 * tiles_n, first_m = (t / gsize) * 4, gm = min(4, tiles_m - first_m);
+  const int m0 = (first_m + (t % gsize) % gm) * BM, n0 = ((t % gsize) / gm) * ON;
+
+  const float* X = static_cast<const float*>(p.x);
+  const float* W = static_cast<const float*>(p.w);
+  const float* W2 = static_cast<const float*>(p.w2);
+  // Chunk i of a thread: sub-stage sub[i], row r of [x rows | weight rows],
+  // columns 8 (tid % 4) .. + 7.  A SwiGLU tile's 16-row weight blocks
+  // alternate gate and up rows of the same 16 outputs.
+  const int c4 = tid & 3;
+  auto chunk = [&](int i, int& sub, int& row) {
+    const int ci = i * NT + wave * 64;  // uniform part
+    sub = ci / CPS;
+    row = (ci % CPS) / 4 + (lane >> 2);
+  };
+  // each through a buffer resource over the tile's rows of its operand
+  uint32_t voff[CH];  // byte offset of the chunk at stage 0
+  __amdgpu_buffer_rsrc_t rs[CH];
+#pragma unroll
+  for (int i = 0; i < CH; ++i) {
+    int sub, row;
+    chunk(i, sub, row);
+    const int first = ((i * NT + wave * 64) % CPS) / 4;  // the wave's first row names the operand
+    const bool is_x = first < BM;
+    const int64_t ld = is_x ? p.ldx : p.ldw;
+    const int base = is_x ? m0 : n0, rows = is_x ? p.M - m0 : p.N - n0;
+    const float* op = is_x ? X : EPI == 2 && ((first - BM) & 16) ? W2 : W;
+    const int rb = row - BM;
+    const int r = min(is_x ? row : EPI == 2 ? (rb >> 5) * 16 + (rb & 15) : rb, rows - 1);
+    rs[i] = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(op + base * ld), 0,
+                                              static_cast<int>(min(rows, BM + BN) * (int)ld * 4), 0x00020000);
+    voff[i] = (uint32_t)(r * (int)ld + sub * 32 + 8 * c4) * 4u;
+  }
+  const int nsub = (p.K + 31) / 32, nst = (nsub + U - 1) / U;
+  float4_t ld[D][CH][2];
+  auto load = [&](int st, int d) {
+    const bool whole = (st + 1) * U * 32 <= p.K;
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+      int sub, row;
+      chunk(i, sub, row);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        uint32_t vo = voff[i] + 16 * h;
+        const uint32_t so = (uint32_t)st * (U * 128);
+        if (!whole) {  // past K: the row's last four elements, zeroed by split()
+          const int k = st * U * 32 + sub * 32 + 8 * c4 + 4 * h;
+          vo -= k + 4 > p.K ? (uint32_t)(k - (p.K - 4)) * 4u : 0u;
+        }
+        const uint4_t v = __builtin_amdgcn_raw_buffer_load_b128(rs[i], whole ? vo : vo + so, whole ? so : 0u, 0);
+        ld[d][i][h] = __builtin_bit_cast(float4_t, v);
+      }
+    }
+  };
+  // LDS: per buffer, sub-stage and plane [x rows | weight rows][32] bf16, the
+  // 16-byte chunk c of row r at c ^ ((r >> 2) & 3) (16 consecutive rows of
+  // one chunk, and 4 rows of all four, cover the 64 banks once)
+  uint32_t smallest = 0xffffffffu;  // of |x| > 0, as 2 * bits - 1
+  auto split = [&](int st, int d) {
+    const bool whole = (st + 1) * U * 32 <= p.K;
+    __bf16* const buf = smem + (st & 1) * kBuf;
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+      int sub, row;
+      chunk(i, sub, row);
+      float4_t a = ld[d][i][0], b = ld[d][i][1];
+      if (!whole) {
+        const int k = st * U * 32 + sub * 32 + 8 * c4;
+        if (k >= p.K) a = float4_t{0.f, 0.f, 0.f, 0.f};
+        if (k + 4 >= p.K) b = float4_t{0.f, 0.f, 0.f, 0.f};
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        smallest = min(smallest, 2u * __float_as_uint(a[e]) - 1u);
+        smallest = min(smallest, 2u * __float_as_uint(b[e]) - 1u);
+      }
+      bf16x8 hi, mid, lo;
+      split8(a, b, hi, mid, lo);
+      __bf16* const dst = buf + sub * kSub + row * 32 + ((c4 ^ ((row >> 2) & 3)) << 3);
+      *reinterpret_cast<bf16x8*>(dst) = hi;
+      *reinterpret_cast<bf16x8*>(dst + kPlane) = mid;
+      *reinterpret_cast<bf16x8*>(dst + 2 * kPlane) = lo;
+    }
+  };
+
+  // 16 x 16 x 32 products, weights as the A operand (a lane's four results
+  // are consecutive columns of one row).  Six products per block: all but
+  // mid*lo, lo*mid and lo*lo, at most 2^-26 of the term; the small ones first.
+  // Each 32-deep step starts from zero, so the small products are summed
+  // among themselves.
+  const bool active = wave < VM * VN;
+  float4_t sum[TM][TN], tot[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) sum[i][j] = tot[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+  const int r16 = lane & 15, c16 = lane >> 4;
+  const int goff = r16 * 32 + ((c16 ^ ((r16 >> 2) & 3)) << 3);
+  auto product = [&](const __bf16* sub) {
+    const __bf16* ab = sub + wm * WM * 32 + goff;
+    const __bf16* bb = sub + (BM + wn * WN) * 32 + goff;
+    bf16x8 bf[TN][3];
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int s = 0; s < 3; ++s) bf[j][s] = *reinterpret_cast<const bf16x8*>(bb + s * kPlane + j * 512);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      bf16x8 af[3];
+#pragma unroll
+      for (int s = 0; s < 3; ++s) af[s] = *reinterpret_cast<const bf16x8*>(ab + s * kPlane + i * 512);
+      constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+      float4_t acc[TN];
+#pragma unroll
+      for (int q = 0; q < 6; ++q)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              bf[j][pb[q]], af[pa[q]], q == 0 ? float4_t{0.f, 0.f, 0.f, 0.f} : acc[j], 0, 0, 0);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) sum[i][j] += acc[j];
+    }
+  };
+  constexpr int G = 4;  // steps added up before they join the running sum
+  auto fold = [&] {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        tot[i][j] += sum[i][j];
+        sum[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+      }
+  };
+  auto compute = [&](int st) {
+    const __bf16* const buf = smem + (st & 1) * kBuf;
+    if (!active) return;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      product(buf + u * kSub);  // sub-stages past K are zeros
+      if ((st * U + u) % G == G - 1) fold();
+    }
+  };
+
+  if (tid == 0) tiny_flag = 0;
+  load(0, 0);
+  if (D == 2 && nst > 1) load(1, 1);
+  split(0, 0);
+  if (nst > D) load(D, 0);
+  lds_barrier();
+  // stage st is multiplied from one buffer while stage st + 1 (in registers
+  // since D stages) is split into the other
+  auto step = [&](int st, int d) {
+    if (st + 1 < nst) {
+      split(st + 1, d);
+      if (st + 1 + D < nst) load(st + 1 + D, d);
+    }
+    compute(st);
+    lds_barrier();
+  };
+  int st = 0;
+  if constexpr (FAST) {
+    // whole stages with two more after them: one basic block, so that the
+    // splitting of stage st + 1 runs under the products of stage st
+    const int nfast = min(nst - 2, p.K / 32 - 2);
+    auto fast = [&](int s, __bf16* cur, __bf16* oth) {
+      const __bf16* ab = cur + wm * WM * 32 + goff;
+      const __bf16* bb = cur + (BM + wn * WN) * 32 + goff;
+      bf16x8 bf[TN][3];
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) bf[j][q] = *reinterpret_cast<const bf16x8*>(bb + q * kPlane + j * 512);
+      bf16x8 pl[CH][3];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        bf16x8 af[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) af[q] = *reinterpret_cast<const bf16x8*>(ab + q * kPlane + i * 512);
+        constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+        float4_t acc[TN];
+#pragma unroll
+        for (int q = 0; q < 6; ++q)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                bf[j][pb[q]], af[pa[q]], q == 0 ? float4_t{0.f, 0.f, 0.f, 0.f} : acc[j], 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) sum[i][j] += acc[j];
+      }
+#pragma unroll
+      for (int i = 0; i < CH; ++i) {
+        int sub, row;
+        chunk(i, sub, row);
+        const float4_t a = ld[0][i][0], b = ld[0][i][1];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          smallest = min(smallest, 2u * __float_as_uint(a[e]) - 1u);
+          smallest = min(smallest, 2u * __float_as_uint(b[e]) - 1u);
+        }
+        split8(a, b, pl[i][0], pl[i][1], pl[i][2]);
+        __bf16* const dst = oth + sub * kSub + row * 32 + ((c4 ^ ((row >> 2) & 3)) << 3);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) *reinterpret_cast<bf16x8*>(dst + q * kPlane) = pl[i][q];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          ld[0][i][h] = __builtin_bit_cast(
+              float4_t, __builtin_amdgcn_raw_buffer_load_b128(rs[i], voff[i] + 16 * h, (uint32_t)(s + 2) * 128u, 0));
+        }
+      }
+      __builtin_amdgcn_sched_group_barrier(0x100, 3 * TN + 3, 0);
+#pragma unroll
+      for (int q = 0; q < 6 * TM * TN; ++q) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+        if (q % (2 * TN) == 0) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        if (q % 10 == 9) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      lds_barrier();
+    };
+    for (; st + 1 < nfast; st += 2) {
+      fast(st, smem, smem + kBuf);
+      fast(st + 1, smem + kBuf, smem);
+      if ((st + 1) % G == G - 1) fold();
+    }
+  }
+  if constexpr (D == 1) {
+    for (; st < nst; ++st) step(st, 0);
+  } else {
+    for (; st < nst; st += 2) {
+      step(st, 1);
+      if (st + 1 < nst) step(st + 1, 0);
+    }
+  }
+  if (active) fold();
+
+  // Values the split does not hold: below 2^-100 the low parts leave bf16's
+  // range; infinities, NaN and values that round to infinity make every
+  // output they meet NaN.  Such tiles are formed again on f32 products.
+  if (smallest < (27u << 24) - 1u) tiny_flag = 1;
+  lds_barrier();
+  if (!active) return;
+  bool again = tiny_flag != 0;
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) again |= !(fabsf(tot[i][j][e]) < __builtin_inff());
+  again = __ballot(again) != 0;
+
+  const int esz = (EPI == 1 || p.dtype_out != 1) ? 4 : 2;
+  const bool yvec = ((reinterpret_cast<uintptr_t>(p.y) | (uintptr_t)(p.ldy * esz)) & (4 * esz - 1)) == 0;
+  const int orow = m0 + wm * WM + r16, ocol = n0 + wn * (EPI == 2 ? WN / 2 : WN) + 4 * c16;
+  constexpr int TO = EPI == 2 ? TN / 2 : TN;
+  auto finish = [&](int i, int j, float4_t v, const float4_t& up) {
+    const int r = orow + 16 * i, c = ocol + 16 * j;
+    if constexpr (EPI == 2) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (p.dtype_out == 1) {
+          const float gh = static_cast<float>(to_f16(v[e]));
+          const float sh = static_cast<float>(to_f16(silu_hw(gh)));
+          v[e] = sh * static_cast<float>(to_f16(up[e]));
+        } else {
+          v[e] = (v[e] / (1.0f + expf(-v[e]))) * up[e];
+        }
+      }
+      store_row4(p, r, c, v, yvec);
+    } else if constexpr (EPI == 1) {
+      if (r >= p.M) return;
+      float* dst = static_cast<float*>(p.y) + (int64_t)r * p.ldy + c;
+      auto rd = [&](float x) { return p.dtype_out == 1 ? static_cast<float>(static_cast<half_t>(x)) : x; };
+      if (yvec && c + 3 < p.N) {
+        float4_t h = *reinterpret_cast<const float4_t*>(dst);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) h[e] += rd(v[e]);
+        *reinterpret_cast<float4_t*>(dst) = h;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (c + e < p.N) dst[e] += rd(v[e]);
+      }
+    } else {
+      store_row4(p, r, c, v, yvec);
+    }
+  };
+  if (!again) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TO; ++j)
+        finish(i, j, tot[i][EPI == 2 ? 2 * j : j], tot[i][EPI == 2 ? 2 * j + 1 : j]);
+    return;
+  }
+  // one 16 x 16 block on v_mfma_f32_16x16x4_f32, operands straight from memory
+  auto exact = [&](const float* w, int xr, int wr) __attribute__((always_inline)) {
+    float4_t s = {0.f, 0.f, 0.f, 0.f};
+    const float* xp = X + (int64_t)min(xr + r16, p.M - 1) * p.ldx;
+    const float* wp = w + (int64_t)min(wr + r16, p.N - 1) * p.ldw;
+    for (int k0 = 0; k0 < p.K; k0 += 32) {
+      float4_t a = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+        const int k = k0 + 16 * kb + 4 * c16;
+        float4_t xv = {0.f, 0.f, 0.f, 0.f}, wv = xv;
+        if (k < p.K) {
+          xv = *reinterpret_cast<const float4_t*>(xp + k);
+          wv = *reinterpret_cast<const float4_t*>(wp + k);
+        }
+        Mma<float>::mma(a, wv, xv);
+      }
+      s += a;
+    }
+    return s;
+  };
+  for (int i = 0; i < TM; ++i)
+    for (int j = 0; j < TO; ++j) {
+      const int xr = m0 + wm * WM + 16 * i, wr = ocol - 4 * c16 + 16 * j;
+      const float4_t v = exact(W, xr, wr);
+      finish(i, j, v, EPI == 2 ? exact(W2, xr, wr) : v);
+    }
+}
+
+}  // namespace
+}  // namespace clef

@@ -260,3 +260,57 @@ def test_gemm_small_tiles_write_only_their_rows(clef):
     clef.gemm(x, w, out=buf[:M, 8:8 + N])
     _check_f16(buf[:M, 8:8 + N], x, w)
     assert (buf[M:] == 7).all() and (buf[:, :8] == 7).all() and (buf[:, 8 + N:] == 7).all()
+
+
+# f32 operands with 16-byte rows: each tile shape (32 x 32 .. 256 x 128), edges
+# and remainders in rows and columns, K of one float4, below one step, ragged
+# steps and stages
+F32_SPLIT = [(1, 16, 4), (31, 33, 28), (33, 100, 196), (1, 2048, 6144), (65, 2047, 132), (300, 2048, 1028),
+             (500, 8192, 96), (129, 4099, 64), (2048, 8192, 256), (1100, 9216, 100)]
+
+
+@gpu
+@pytest.mark.parametrize("M,N,K", F32_SPLIT)
+def test_gemm_f32_split_tiles(clef, M, N, K):
+    """The split forms each product to 2^-26 of the term and rounds a sum at
+    most twice per 32 columns: |err| <= (2^-25 + (6 + K / 16) 2^-24) sum|x w|."""
+    x, w = _inputs(31, M, N, K, torch.float32)
+    _, u = _inputs(32, 1, N, K, torch.float32)
+    ref, scale = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    bound = (2.0 ** -25 + (6 + K / 16) * 2.0 ** -24) * scale
+    y = clef.gemm(x, w)
+    assert ((y.double() - ref).abs() <= bound).all()
+    # in the 2-norm the error of a random sum is far smaller: below that of the
+    # f32 MFMA kernel (1.0e-7 at K = 36, 2.7e-7 at K = 6144)
+    assert (y.double() - ref).norm() <= 2e-7 * ref.norm()
+    h0 = torch.randn((M, N), device="cuda")
+    assert torch.equal(clef.gemm(x, w, residual=h0.clone()), h0 + y)
+    assert torch.equal(clef.gemm(x, w, out_dtype=torch.float16), y.half())
+    g, v = y, clef.gemm(x, u)
+    s = clef.gemm_swiglu(x, w, u)
+    assert torch.allclose(s, g / (1 + torch.exp(-g)) * v, rtol=2e-6, atol=1e-30)
+    # a row does not depend on how many share the call
+    xl = torch.cat([x, torch.zeros((4096, K), device="cuda")])
+    assert torch.equal(clef.gemm(xl, w)[:M], y)
+
+
+@gpu
+@pytest.mark.parametrize("M", [20, 150, 300, 2048])
+def test_gemm_f32_split_special_values(clef, M):
+    """Infinities, NaN, values next to the largest float and far below 2^-100
+    give what an f32 product gives."""
+    N, K = 8192, 64
+    x, w = _inputs(33, M, N, K, torch.float32)
+    x[3, 5], x[7, 9], x[11, 2], x[12] = float("inf"), float("nan"), 3.4e38, 0.0
+    w[100, 30] = -float("inf")
+    x[13] *= 1e-32
+    x[14] = torch.randn(K, device="cuda") * 1e-38  # subnormal parts
+    w[200] *= 1e20
+    y = clef.gemm(x, w).double()
+    ref = x.double() @ w.double().T
+    ok = ref.abs() <= 3.0e38
+    scale = x.double().abs() @ w.double().abs().T
+    assert ((y - ref).abs()[ok] <= (1e-6 * scale + 2.0 ** -145)[ok]).all()
+    assert torch.equal(torch.isnan(y), torch.isnan(ref))
+    big = ref.abs() > 3.5e38
+    assert torch.isinf(y[big]).all() and torch.equal(y[big].sign(), ref[big].sign())
