@@ -502,9 +502,13 @@ __device__ __forceinline__ void q_prepare(const AttnParams& p, int t, int h, int
   }
 }
 
-template <int D, bool VL>
+// NACT: waves that own queries (16 each).  Items of 128 queries (NACT 8) give a
+// short request too few of them: the waves past NACT then only move keys and
+// values (launch rule below).  A query's products and softmax steps do not
+// depend on NACT.
+template <int D, bool VL, int NACT>
 __global__ __launch_bounds__(512) void attn_f16_w8(AttnParams p) {
-  constexpr int BQ = 128, BK = 64, NW = 8;
+  constexpr int BQ = 16 * NACT, BK = 64, NW = 8;
   constexpr int KS = D / 8;           // 16-byte chunks per key row
   constexpr int NKS = D / 32;         // 32-deep k-steps of S^T = K Q^T
   constexpr int NDT = D / 16;         // 16-row tiles of O^T
@@ -514,6 +518,7 @@ __global__ __launch_bounds__(512) void attn_f16_w8(AttnParams p) {
   constexpr int PD = 4;               // LDS fragment reads in flight ahead of the MFMAs
   static_assert(D == 256 || D == 128, "head width");
   static_assert(NDK >= 1 && NDV >= 1, "whole DMA instructions per wave");
+  static_assert(NACT == 8 || !VL, "ragged batches: items of 128 queries");
 
   __shared__ __attribute__((aligned(1024))) half_t sK[2][BK * D];
   __shared__ __attribute__((aligned(1024))) half_t sV[2][D * BK];
@@ -521,6 +526,7 @@ __global__ __launch_bounds__(512) void attn_f16_w8(AttnParams p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 15, g = lane >> 4;
+  const bool active = NACT == NW || wave < NACT;
 
   // work items dealt as in attn_f16 (longest first, boustrophedon); a ragged
   // batch's items are its (sequence, query tile) pairs, ranked by key count
@@ -557,7 +563,7 @@ __global__ __launch_bounds__(512) void attn_f16_w8(AttnParams p) {
 
   // Q^T fragments (B operand): lane (n, g) holds d = 32 s + 8 g .. + 7 of its query
   half8 qf[NKS];
-  {
+  if (active) {
     const int r = min(q0 + 16 * wave + n, qn - 1);
     bool prepared = false;
     if constexpr (!VL) {
@@ -684,7 +690,7 @@ __global__ __launch_bounds__(512) void attn_f16_w8(AttnParams p) {
   lds_barrier();
   float4_t Sc[4], Sn[4];
   half8 fb[PD];
-  {
+  if (active) {
     const char* kbase = reinterpret_cast<const char*>(sK[0]);
 #pragma unroll
     for (int t = 0; t < 4; ++t) Sc[t] = float4_t{0.f, 0.f, 0.f, 0.f};
@@ -697,8 +703,8 @@ __global__ __launch_bounds__(512) void attn_f16_w8(AttnParams p) {
       __builtin_amdgcn_sched_barrier(0);
     }
   }
-  float m_ref;
-  {
+  float m_ref = 0.0f;
+  if (active) {
     float mx = -INFINITY;
 #pragma unroll
     for (int t = 0; t < 4; ++t)
@@ -735,6 +741,11 @@ __global__ __launch_bounds__(512) void attn_f16_w8(AttnParams p) {
         }
       }
       lds_barrier();
+    }
+    if (NACT < NW && !active) {
+      vm_wait_all();
+      lds_barrier();
+      return;
     }
     const char* kbase = reinterpret_cast<const char*>(sK[(j + 1) & 1]);
     const char* vbase = reinterpret_cast<const char*>(sV[j & 1]);
@@ -829,6 +840,10 @@ __global__ __launch_bounds__(512) void attn_f16_w8(AttnParams p) {
     }
     return r;
   };
+  if (NACT < NW && !active) {
+    if (p.vec_io == 2) lds_barrier();
+    continue;
+  }
   if (p.vec_io == 2) {
     // 16-byte gate and output rows: round(O / l) of the wave's 16 queries is
     // staged in LDS (free after the last key tile; waves 0-3 in sK, 4-7 in
@@ -958,6 +973,32 @@ int launch(const AttnParams& p0, hipStream_t s) {
 
 // the single-sequence core at two waves per SIMD
 constexpr bool kW8 = true;
+
+// resident work-groups (CUs x occupancy) of an instance, per device: the
+// ragged instance carries the prefix-segment logic and may fit fewer per CU,
+// and a grid above the resident count would lose the longest-first item order
+template <int D, bool VL, int NACT>
+int resident_w8() {
+  static int cached[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
+  if (cached[dev] == 0) {
+    int cus = 0, per = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, attn_f16_w8<D, VL, NACT>, 512, 0) != hipSuccess || per <= 0)
+      per = 1;
+    cached[dev] = cus * per;
+  }
+  return cached[dev];
+}
+
+template <int D, bool VL, int NACT>
+int launch_w8_items(const AttnParams& p, int qtiles, hipStream_t s) {
+  const int items = qtiles * p.heads, resident = resident_w8<D, VL, NACT>();
+  hipLaunchKernelGGL((attn_f16_w8<D, VL, NACT>), dim3(items < resident ? items : resident), dim3(512), 0, s, p);
+  return check_launch("attention");
+}
+
 template <int D>
 int launch_w8(const AttnParams& p0, hipStream_t s) {
   AttnParams p = p0;
@@ -967,30 +1008,17 @@ int launch_w8(const AttnParams& p0, hipStream_t s) {
   if (p.vec_io && ((reinterpret_cast<uintptr_t>(p.gate) | reinterpret_cast<uintptr_t>(p.y)) & 15) == 0 &&
       p.ldg % 8 == 0 && p.hsg % 8 == 0 && p.ldy % 8 == 0 && p.d == D)
     p.vec_io = 2;
-  // resident work-groups (CUs x occupancy) of the instance launched, per
-  // device: the ragged instance carries the prefix-segment logic and may fit
-  // fewer per CU, and a grid above the resident count would lose the
-  // longest-first item order
-  static int cached[64][2] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-  const int vl = p.cu_q ? 1 : 0;
-  if (cached[dev][vl] == 0) {
-    int cus = 0, per = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
-    const hipError_t e = vl ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, attn_f16_w8<D, true>, 512, 0)
-                            : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, attn_f16_w8<D, false>, 512, 0);
-    if (e != hipSuccess || per <= 0) per = 1;
-    cached[dev][vl] = cus * per;
-  }
-  const int qtiles = p.cu_q ? (p.qn + 127) / 128 + p.nseq : (p.qn + 127) / 128;
-  const int items = qtiles * p.heads;
-  const int groups = items < cached[dev][vl] ? items : cached[dev][vl];
-  if (p.cu_q)
-    hipLaunchKernelGGL((attn_f16_w8<D, true>), dim3(groups), dim3(512), 0, s, p);
-  else
-    hipLaunchKernelGGL((attn_f16_w8<D, false>), dim3(groups), dim3(512), 0, s, p);
-  return check_launch("attention");
+  if (p.cu_q) return launch_w8_items<D, true, 8>(p, (p.qn + 127) / 128 + p.nseq, s);
+  // Items of 128 queries that do not even fill the CUs once: 64 queries each
+  // (one multiplying wave per SIMD: a key tile takes ~1.0 instead of ~2.3 us).
+  // 16 heads, us on 128 -> on 64: 100 queries behind 512 keys 28.3 -> 20.4,
+  // 777 behind 256 39.2 -> 29.3, 1500 52.6 -> 39.3, 2048 (256 items) 68.4 ->
+  // 58.6; above, 128 wins: 3000 103 against 120, 4096 163 against 203.  (Items
+  // of 32 or 16 gain at most 1 us more, below 400 queries, and lose from there.)
+  const int qtiles = (p.qn + 127) / 128;
+  if ((int64_t)qtiles * p.heads <= resident_w8<D, false, 8>())
+    return launch_w8_items<D, false, 4>(p, (p.qn + 63) / 64, s);
+  return launch_w8_items<D, false, 8>(p, qtiles, s);
 }
 
 }  // namespace

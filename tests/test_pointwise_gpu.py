@@ -350,3 +350,20 @@ def test_attention_varlen_matches_per_sequence_oracle(clef, np_, d):
         sig = 1.0 / (1.0 + np.exp(-g[a:b].reshape(b - a, heads * d).astype(np.float64)))
         exp = att.astype(np.float16).astype(np.float64) * sig.astype(np.float16).astype(np.float64)
         np.testing.assert_allclose(y[a:b], exp, rtol=1e-2, atol=5e-3)
+
+
+@gpu
+@pytest.mark.parametrize("qn,kn", [(1, 1), (1, 70), (63, 63), (64, 64), (65, 100), (100, 612), (700, 701), (2048, 2048)])
+def test_attention_short_items_equal_long_items(clef, qn, kn):
+    """Short requests run on items of 64 queries, long ones on 128: the first
+    queries of a 2200-query call (items of 128) over the same keys, bit for bit."""
+    heads, kvh, d, big = 16, 2, 256, 2200
+    gen = torch.Generator(device="cuda").manual_seed(41)
+    rnd = lambda *s: torch.randn(s, generator=gen, device="cuda").half()
+    off = kn - qn
+    q, k, v, gate = rnd(heads, big, d), rnd(kvh, off + big, d), rnd(off + big, kvh * d), rnd(big, heads, d)
+    vt = clef.values_transposed(v, kvh, d)
+    long = clef.attention_gated(q, k, vt, gate)
+    short = clef.attention_gated(q[:, :qn].contiguous(), k[:, :kn].contiguous(),
+                                 clef.values_transposed(v[:kn], kvh, d), gate[:qn])
+    assert torch.equal(short, long[:qn])
