@@ -94,13 +94,13 @@ struct Row8<float> {
 
 
 // Vectorised conv + SiLU: 8 consecutive channels per thread and a run of
-// kConvRun tokens (taps <= 4; T4: taps == 4 known at compile time).  The
-// run's kConvRun + 3 input rows are all requested before the first product,
-// so a thread keeps that many 16-byte loads in flight; rows before token 0
-// come from the f32 history.  Only the first run (t0 = 0) can reach before
-// the history, so the others are compiled without the per-tap checks.
+// RUN tokens (taps <= 4; T4: taps == 4 known at compile time).  The run's
+// RUN + 3 input rows are all requested before the first product, so a thread
+// keeps that many 16-byte loads in flight; rows before token 0 come from the
+// f32 history.  Only the first run (t0 = 0) can reach before the history, so
+// the others are compiled without the per-tap checks.
 constexpr int kConvRun = 16;
-template <class TI, class TO, bool T4>
+template <class TI, class TO, bool T4, int RUN>
 __global__ __launch_bounds__(256) void conv_silu_vec_kernel(const TI* __restrict__ x, int64_t ldx,
                                                             const float* __restrict__ hist, int hrows,
                                                             const float* __restrict__ w, int taps_rt,
@@ -108,8 +108,9 @@ __global__ __launch_bounds__(256) void conv_silu_vec_kernel(const TI* __restrict
   const int c0 = (blockIdx.x * 256 + threadIdx.x) * 8;
   if (c0 >= W) return;
   const int taps = T4 ? 4 : taps_rt;
-  const int t0 = blockIdx.y * kConvRun;
-  constexpr int R = kConvRun + 3;
+  const int t0 = blockIdx.y * RUN;
+  static_assert(RUN >= 3, "only the first run reaches the history");
+  constexpr int R = RUN + 3;
   Row8<TI> raw[R];  // raw[r]: token t0 - 3 + r
 #pragma unroll
   for (int r = 0; r < R; ++r) {
@@ -148,7 +149,7 @@ __global__ __launch_bounds__(256) void conv_silu_vec_kernel(const TI* __restrict
   auto run = [&](auto edge) {
     constexpr bool EDGE = decltype(edge)::value;
 #pragma unroll
-    for (int u = 0; u < kConvRun; ++u) {
+    for (int u = 0; u < RUN; ++u) {
       const int t = t0 + u;
       if (t >= T) break;
       TO out[8];
@@ -790,10 +791,22 @@ __global__ __launch_bounds__(256) void embed_vec_kernel(const int32_t* __restric
   *reinterpret_cast<float4_t*>(dst + 4) = b;
 }
 
-__global__ __launch_bounds__(64) void head_kernel(const float* x, int H, const float* w, float* logits) {
+// One logit per wave, sums over features lane, lane + 64, ...: a chain of H / 64
+// adds, fed by 16 loads of each operand at a time (a 2048-wide logit took 16
+// us with one load in flight, 2.0 now: latency, not bytes).
+__global__ __launch_bounds__(64) void head_kernel(const float* __restrict__ x, int H, const float* __restrict__ w,
+                                                  float* __restrict__ logits) {
   const int j = blockIdx.x, lane = threadIdx.x;
   float s = 0.0f;
-  for (int i = lane; i < H; i += 64) s += x[i] * w[(int64_t)j * H + i];
+  int i = lane;
+  for (; i + 15 * 64 < H; i += 16 * 64) {
+    float a[16], b[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) a[u] = x[i + 64 * u], b[u] = w[(int64_t)j * H + i + 64 * u];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) s += a[u] * b[u];
+  }
+  for (; i < H; i += 64) s += x[i] * w[(int64_t)j * H + i];
   s = wave_sum(s);
   if (lane == 0) logits[j] = s;
 }
@@ -860,16 +873,29 @@ extern "C" int clef_conv_silu(const void* x, int64_t ldx, int dtype_in, const fl
   const bool vec = taps <= 4 && W % 8 == 0 && ldx % 8 == 0 && ldy % 8 == 0 &&
                    (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0;
   if (vec) {
-    const dim3 g((W / 8 + 255) / 256, (T + kConvRun - 1) / kConvRun);
+    // Runs of 16 tokens re-read 3 rows in 19, but a short request gives them
+    // too few work-groups, each waiting on 19 loads: runs of 4 up to 100
+    // work-groups, f16 runs of 8 up to 512.  W = 8192, us on 16 / 8 / 4 tokens:
+    // T = 100 f16 8.9 / 6.1 / 4.7, f32 8.8 / 6.3 / 5.1; 400 f16 9.9 / 7.0 / 6.9,
+    // f32 10.0 / 8.0 / 8.6; 1000 f16 11.0 / 10.7 / 11.4, f32 14.2 / 16.2 / 17.6;
+    // 1500 f16 17.2 / 14.2 / 14.8 (4096 in a prefill: 16 wins).
+    const int gx = (W / 8 + 255) / 256;
+    const int64_t groups = (int64_t)gx * ((T + kConvRun - 1) / kConvRun);
+    const int run = taps != 4 ? kConvRun : groups <= 100 ? 4 : dtype_in == CLEF_F16 && groups <= 512 ? 8 : kConvRun;
+    const dim3 g(gx, (T + run - 1) / run);
     hipStream_t st = static_cast<hipStream_t>(stream);
-#define CLEF_CONV_VEC(TI, TO, T4)                                                                       \
-  hipLaunchKernelGGL((conv_silu_vec_kernel<TI, TO, T4>), g, dim3(256), 0, st, static_cast<const TI*>(x), ldx, \
+#define CLEF_CONV_VEC(TI, TO, T4, RUN)                                                                       \
+  hipLaunchKernelGGL((conv_silu_vec_kernel<TI, TO, T4, RUN>), g, dim3(256), 0, st, static_cast<const TI*>(x), ldx, \
                      history, history_rows, w, taps, static_cast<TO*>(y), ldy, T, W)
-#define CLEF_CONV_VEC_T(TI, TO)    \
-  if (taps == 4)                   \
-    CLEF_CONV_VEC(TI, TO, true);   \
-  else                             \
-    CLEF_CONV_VEC(TI, TO, false)
+#define CLEF_CONV_VEC_T(TI, TO)             \
+  if (taps == 4 && run == 4)                \
+    CLEF_CONV_VEC(TI, TO, true, 4);         \
+  else if (taps == 4 && run == 8)           \
+    CLEF_CONV_VEC(TI, TO, true, 8);         \
+  else if (taps == 4)                       \
+    CLEF_CONV_VEC(TI, TO, true, kConvRun);  \
+  else                                      \
+    CLEF_CONV_VEC(TI, TO, false, kConvRun)
     if (dtype_in == CLEF_F16 && dtype_out == CLEF_F16) {
       CLEF_CONV_VEC_T(half_t, half_t);
     } else if (dtype_in == CLEF_F16) {

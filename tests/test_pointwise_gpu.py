@@ -367,3 +367,45 @@ def test_attention_short_items_equal_long_items(clef, qn, kn):
     short = clef.attention_gated(q[:, :qn].contiguous(), k[:, :kn].contiguous(),
                                  clef.values_transposed(v[:kn], kvh, d), gate[:qn])
     assert torch.equal(short, long[:qn])
+
+
+@gpu
+@pytest.mark.parametrize("dt", [torch.float16, torch.float32])
+@pytest.mark.parametrize("T", [1, 2, 3, 4, 5, 17, 400, 401, 2047, 2049])
+@pytest.mark.parametrize("hist", [0, 1, 3])
+def test_conv_short_runs_equal_long_runs(clef, dt, T, hist):
+    """Short calls run 4 or 8 tokens per thread, long ones 16: the first rows of
+    a 3000-token call, bit for bit."""
+    W = 8192
+    gen = torch.Generator(device="cuda").manual_seed(51)
+    x = torch.randn((3000, W), generator=gen, device="cuda").to(dt)
+    w = torch.randn((W, 4), generator=gen, device="cuda")
+    h = torch.randn((hist, W), generator=gen, device="cuda") if hist else None
+    long = clef.conv_silu(x, w, h, out_dtype=dt)
+    assert torch.equal(clef.conv_silu(x[:T], w, h, out_dtype=dt), long[:T])
+
+
+@gpu
+@pytest.mark.parametrize("Hv", [16, 32, 64])
+def test_delta_gates_proj_split_over_outputs_equals_whole(clef, Hv):
+    """Few tokens: a work-group per 16 outputs; many: one for all of them."""
+    K, big = 2048, 2500
+    gen = torch.Generator(device="cuda").manual_seed(52)
+    x = torch.randn((big, K), generator=gen, device="cuda").half()
+    packed = clef.delta_gates_pack((torch.randn((2 * Hv, K), generator=gen, device="cuda") * 0.05).half())
+    dt, alog = torch.randn(Hv, generator=gen, device="cuda"), torch.randn(Hv, generator=gen, device="cuda")
+    g, beta = clef.delta_gates_proj(x, packed, Hv, dt, alog)
+    for T in (1, 15, 16, 17, 500):
+        gs, bs = clef.delta_gates_proj(x[:T], packed, Hv, dt, alog)
+        assert torch.equal(gs, g[:T]) and torch.equal(bs, beta[:T])
+
+
+@gpu
+@pytest.mark.parametrize("H", [1, 63, 64, 1023, 1024, 2048, 2100])
+def test_head_logits_match_f64(clef, H):
+    gen = torch.Generator(device="cuda").manual_seed(53)
+    x, w = torch.randn(H, generator=gen, device="cuda"), torch.randn((5, H), generator=gen, device="cuda")
+    ref = w.double() @ x.double()
+    # a chain of H / 64 adds and six butterfly steps: (H / 64 + 7) 2^-24 of the terms
+    bound = (H / 64 + 8) * 2.0 ** -24 * (w.double().abs() @ x.double().abs())
+    assert ((clef.head_logits(x, w).double() - ref).abs() <= bound).all()
