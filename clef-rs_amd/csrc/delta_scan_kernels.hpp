@@ -265,6 +265,8 @@ __global__ __launch_bounds__(64 * kPW, (sizeof(CT) == 4 && DK > 64) ? 2 : 4) voi
 
   const int chunk = blockIdx.x, hk = blockIdx.y;
   const int rep = p.Hv / p.Hk;
+  // (short scans: gridDim.z work-groups share a k-head's v-heads)
+  const int vpw = rep / static_cast<int>(gridDim.z), v0 = vpw * static_cast<int>(blockIdx.z), v1 = v0 + vpw;
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
   const int col = lane & 15, grp = lane >> 4;
   int t0, n;
@@ -276,7 +278,7 @@ __global__ __launch_bounds__(64 * kPW, (sizeof(CT) == 4 && DK > 64) ? 2 : 4) voi
   // ---- 1. loads: q/k rows (clamped), g and beta of the first v-head
   uint32_t gbits = 0, bbits = 0;
   if (wave == 0) {
-    const int64_t gi = (int64_t)(t0 + min(lane, n - 1)) * p.sgb + (int64_t)hk * rep;
+    const int64_t gi = (int64_t)(t0 + min(lane, n - 1)) * p.sgb + (int64_t)hk * rep + v0;
     gbits = load_bits(p.g, gi, p.dtype_gb);
     bbits = load_bits(p.beta, gi, p.dtype_gb);
   }
@@ -349,7 +351,7 @@ __global__ __launch_bounds__(64 * kPW, (sizeof(CT) == 4 && DK > 64) ? 2 : 4) voi
   }
 
   // ---- 3. per v-head
-  for (int v = 0; v < rep; ++v) {
+  for (int v = v0; v < v1; ++v) {
     const int h = hk * rep + v;
     uint32_t gnext = 0, bnext = 0;
     const int64_t cv = (int64_t)chunk * p.Hv + h;
@@ -359,7 +361,7 @@ __global__ __launch_bounds__(64 * kPW, (sizeof(CT) == 4 && DK > 64) ? 2 : 4) voi
     if (wave == 0) {
       const float gv = lane < n ? bits_to_f32(gbits, p.dtype_gb) : 0.0f;
       const float bv = lane < n ? bits_to_f32(bbits, p.dtype_gb) : 0.0f;
-      if (v + 1 < rep) {  // next v-head's g and beta, awaited at the end of this one
+      if (v + 1 < v1) {  // next v-head's g and beta, awaited at the end of this one
         const int64_t gi = (int64_t)(t0 + min(lane, n - 1)) * p.sgb + h + 1;
         gnext = load_bits(p.g, gi, p.dtype_gb);
         bnext = load_bits(p.beta, gi, p.dtype_gb);
@@ -1239,7 +1241,13 @@ __global__ __launch_bounds__((Carry<CT, IT, DK>::THREADS)) void scan_carry(ScanP
 
 template <class CT, class IT, int DK>
 int launch_dk(const ScanParams& p, hipStream_t stream) {
-  hipLaunchKernelGGL((scan_prepare<CT, IT, DK>), dim3(p.nchunks, p.Hk), dim3(64 * kPW), 0, stream, p);
+  // A work-group prepares a chunk for all v-heads of a k-head, one after the
+  // other; where a work-group per v-head still fits the CUs once, each takes
+  // one (the Gram tiles are formed again).  16 / 32 heads x 128, us: T = 100
+  // f16 14.2 -> 10.8, f32 20.5 -> 15.3; T = 400 16.0 -> 12.6, 23.5 -> 18.4; at
+  // T = 600 (320 work-groups) 16.5 -> 16.0, f32 24.0 -> 30.2.
+  const int vsplit = (int64_t)p.nchunks * p.Hv <= 256 ? p.Hv / p.Hk : 1;
+  hipLaunchKernelGGL((scan_prepare<CT, IT, DK>), dim3(p.nchunks, p.Hk, vsplit), dim3(64 * kPW), 0, stream, p);
   int rc = check_launch("scan_prepare");
   if (rc) return rc;
   const int ntiles = (p.dv + kVT - 1) / kVT;

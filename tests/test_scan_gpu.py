@@ -243,3 +243,21 @@ def test_scan_varlen_matches_per_sequence_oracle(clef, precision, shared):
         eo, _, ef = oracle.delta_scan(qn[a:b], kn[a:b], vn[a:b], gn[a:b], bn[a:b], initial=s0)
         _check(o_all[a:b], eo, precision)
         _check(f_all[s], ef, precision)
+
+
+@gpu
+@pytest.mark.parametrize("precision", ["strict", "mixed"])
+@pytest.mark.parametrize("T", [1, 64, 65, 512])
+def test_short_scan_prepared_per_v_head_equals_long_scan(clef, precision, T):
+    """Short scans prepare each v-head in its own work-group, long ones a
+    k-head's v-heads together: the outputs of a long scan's first tokens and
+    its state captured there, bit for bit (both end on the same chunk grid)."""
+    import workloads
+    x = [t.half() if precision == "mixed" else t for t in workloads.scan_inputs(61, 1024, 16, 32, 128, 128)]
+    scan = clef.DeltaScan(128, 128, precision)
+    out, _, _ = scan.prefill(*x)
+    short, _, final = scan.prefill(*(t[:T] for t in x))
+    assert torch.equal(short, out[:T])
+    if T % 64 == 0:
+        _, captured, _ = scan.prefill(*x, capture=T)
+        assert torch.equal(final, captured)
