@@ -917,7 +917,9 @@ int launch(const GemmParams& p, hipStream_t s) {
   // output and the residual add)
   const bool persistent = EPI != 1 && p.dtype_out == 1 && ntiles > cus && (cus & 7) == 0 && p.K / kBK >= 2;
   if constexpr (BM == 256 && (BN == 256 || (BN != 256 && EPI != 1))) {
-    if constexpr (EPI != 1) {
+    // (a SwiGLU wave of 256 x 192 tiles stores 48 columns a row: not whole
+    // 8-column chunks per lane, so it takes the one-tile form)
+    if constexpr (EPI == 0 || (EPI == 2 && BN != 192)) {
       if (p.dtype_out == 1 && (cus & 7) == 0 && p.K / kBK >= 2) {
         hipLaunchKernelGGL((gemm_f16_w4<EPI, true, BN>), dim3(ntiles < cus ? ntiles : cus), dim3(256), 0, s, p);
         return check_launch("gemm");
@@ -1099,8 +1101,10 @@ bool gemm_f16_dma_ok(const GemmParams& p) {
 // 256 x 256 for N = 12288, 256 x 192 for N = 9216 (768 tiles: 3 full rounds
 // instead of 2.25), 256 x 128 for M = 4096, N = 2048 (256 tiles: one round),
 // 128 x 128 for M = N = 2048 (256 tiles instead of 128 of 256 x 128, which
-// leave half the CUs idle).  SwiGLU keeps widths 256 or 128 (its wave columns
-// pair gate and up blocks).
+// leave half the CUs idle), 256 x 192 for the SwiGLU of 1000 rows (256 tiles:
+// one whole round instead of 192 tiles of 256 x 256; 54.5 -> 51.3 us; 700 rows
+// 59.4 -> 51.4, 3000 155 -> 141; at 1300 rows, where 256 x 128 needs as many
+// rounds x area, it is 4% slower than that, hence its higher cost).
 //
 // The ring kernel's small tiles (gemm_ring.hpp) enter with their measured
 // time of a round in the same unit (1400 per us at K = 2048: 128 x 128 takes
@@ -1131,7 +1135,7 @@ static TileShape gemm_f16_tile_shape(const GemmParams& p, int epilogue) {
     double c;
   };
   const Cand cands[] = {{{256, 256, kRingNone}, cost(256, 256, 1.0)},
-                        {{256, 192, kRingNone}, epilogue == 2 ? 1e300 : cost(256, 192, 1.1)},
+                        {{256, 192, kRingNone}, cost(256, 192, epilogue == 2 ? 1.22 : 1.1)},
                         {{256, 128, kRingNone}, cost(256, 128, 1.2)},
                         {{128, 128, kRingNone}, cost(128, 128, 1.5)},
                         {{128, 64, kRing128x64}, rounds(128, 64) * 20000.0},
@@ -1176,7 +1180,7 @@ int gemm_f16_dma_launch(const GemmParams& p, int epilogue, hipStream_t s) {
     return bn == 256 ? launch<256, 256, 0>(p, s) : bn == 192 ? launch<256, 192, 0>(p, s) : launch<256, 128, 0>(p, s);
   if (epilogue == 1)
     return bn == 256 ? launch<256, 256, 1>(p, s) : bn == 192 ? launch<256, 192, 1>(p, s) : launch<256, 128, 1>(p, s);
-  return bn == 256 ? launch<256, 256, 2>(p, s) : launch<256, 128, 2>(p, s);
+  return bn == 256 ? launch<256, 256, 2>(p, s) : bn == 192 ? launch<256, 192, 2>(p, s) : launch<256, 128, 2>(p, s);
 }
 
 }  // namespace clef

@@ -314,3 +314,14 @@ def test_gemm_f32_split_special_values(clef, M):
     assert torch.equal(torch.isnan(y), torch.isnan(ref))
     big = ref.abs() > 3.5e38
     assert torch.isinf(y[big]).all() and torch.equal(y[big].sign(), ref[big].sign())
+
+
+@gpu
+@pytest.mark.parametrize("M,N,K", [(1000, 6144, 128), (700, 6144, 64), (1024, 6100, 192), (3000, 6144, 64)])
+def test_swiglu_192_wide_tiles(clef, M, N, K):
+    """256 x 192 tiles (96 outputs): whole and ragged rows and columns, one to
+    three K stages; equal to the unfused products."""
+    x, wg = _inputs(25, M, N, K, torch.float16)
+    _, wu = _inputs(26, 1, N, K, torch.float16)
+    y = clef.gemm_swiglu(x, wg, wu)
+    assert torch.equal(y, clef.silu_mul(clef.gemm(x, wg), clef.gemm(x, wu)))
