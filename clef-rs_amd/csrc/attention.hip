@@ -17,6 +17,7 @@
 
 #include "../../include/clef_hip.h"
 #include "attention.hpp"
+#include "bf16_split.hpp"
 #include "common.hpp"
 
 namespace clef {
@@ -24,8 +25,17 @@ namespace {
 
 __device__ __forceinline__ void wave_lds_sync() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
+// LDS of the body below: K tile, V^T tile, and per wave a P tile.
 template <class T, int D>
-__global__ __launch_bounds__(256) void attn_kernel(AttnParams p) {
+constexpr int attn_lds_bytes() {
+  constexpr int EPF = 16 / sizeof(T);
+  return (64 * (D + EPF) + D * (64 + EPF) + 4 * 16 * (64 + EPF)) * (int)sizeof(T);
+}
+
+// 64 query rows of one head, by the first four waves of a work-group (any
+// others only keep its barriers).
+template <class T, int D>
+__device__ __forceinline__ void attn_body(const AttnParams& p, char* smem) {
   constexpr int BQ = 64, BKEY = 64;
   constexpr int EPF = 16 / sizeof(T);
   constexpr int KB = Mma<T>::kBlock;
@@ -36,12 +46,13 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnParams p) {
   typedef typename Mma<T>::frag frag;
   typedef typename Mma<T>::frag vec;  // 16-byte vector of T
 
-  __shared__ __attribute__((aligned(16))) T sK[BKEY * LDK];
-  __shared__ __attribute__((aligned(16))) T sV[D * LDV];
-  __shared__ __attribute__((aligned(16))) T sP[4][16 * LDP];
+  T* const sK = reinterpret_cast<T*>(smem);
+  T* const sV = sK + BKEY * LDK;
+  T* const sP = sV + D * LDV;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bool on = wave < 4;
   const int col = lane & 15, grp = lane >> 4;
   const int qtiles = (p.qn + BQ - 1) / BQ;
   const int h = blockIdx.x % p.heads;
@@ -118,11 +129,18 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnParams p) {
       *reinterpret_cast<vec*>(&sV[r * LDV + c]) = vv;
     }
   };
-  load_tile(0);
-  store_tile(0);
+  if (on) {
+    load_tile(0);
+    store_tile(0);
+  }
   lds_barrier();
   for (int j0 = 0; j0 < key_end; j0 += BKEY) {
     const bool more = j0 + BKEY < key_end;  // uniform over the work-group
+    if (!on) {
+      lds_barrier();
+      if (more) lds_barrier();
+      continue;
+    }
     if (more) load_tile(j0 + BKEY);
 
     // ---- S = Q K^T for 16 rows x 64 keys
@@ -171,7 +189,7 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnParams p) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) O[nt][i] *= rescale[i];
     // ---- P to LDS (accumulator layout -> operand layout)
-    T* P = sP[wave];
+    T* P = sP + wave * (16 * LDP);
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
@@ -194,6 +212,7 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnParams p) {
     }
   }
 
+  if (!on) return;
   // ---- epilogue: y = round(round(O / l) * round(sigmoid(gate)))
   const bool half_out = sizeof(T) == 2;
 #pragma unroll
@@ -218,6 +237,14 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnParams p) {
 }
 
 template <class T, int D>
+__global__ __launch_bounds__(256) void attn_kernel(AttnParams p) {
+  __shared__ __attribute__((aligned(16))) char smem[attn_lds_bytes<T, D>()];
+  attn_body<T, D>(p, smem);
+}
+
+#include "attention_f32.hpp"
+
+template <class T, int D>
 int launch(const AttnParams& p, hipStream_t s) {
   const int qtiles = (p.qn + 63) / 64;
   hipLaunchKernelGGL((attn_kernel<T, D>), dim3(qtiles * p.heads), dim3(256), 0, s, p);
@@ -226,6 +253,9 @@ int launch(const AttnParams& p, hipStream_t s) {
 
 template <class T>
 int launch_d(const AttnParams& p, hipStream_t s) {
+  if constexpr (sizeof(T) == 4) {
+    if (attn_f32_split_ok(p)) return attn_f32_split_launch(p, s);
+  }
   if (p.d <= 32) return launch<T, 32>(p, s);
   if (p.d <= 64) return launch<T, 64>(p, s);
   if (p.d <= 128) return launch<T, 128>(p, s);

@@ -31,15 +31,13 @@
 // 256 x 128 as 2 x 4 waves of 128 x 32: as 4 x 2 of 64 x 64 the second set of
 // sums spills (426 us).
 #pragma once
+#include "bf16_split.hpp"
 #include "common.hpp"
 #include "gemm.hpp"
 
 namespace clef {
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float float2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t uint4_t __attribute__((ext_vector_type(4)));
 
 // Stores four consecutive columns c .. c + 3 of row r, clipped to M x N.
@@ -66,22 +64,6 @@ __device__ __forceinline__ void store_row4(const GemmParams& p, int r, int c, co
       for (int e = 0; e < 4; ++e)
         if (c + e < p.N) dst[e] = o[e];
     }
-  }
-}
-
-// x = hi + mid + lo exactly, each a bf16: round to nearest takes 8 bits, and
-// what is left of a 24-bit significand after two of them fits a third.
-__device__ __forceinline__ void split8(const float4_t& a, const float4_t& b, bf16x8& hi, bf16x8& mid, bf16x8& lo) {
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const float2_t x = e < 2 ? float2_t{a[2 * e], a[2 * e + 1]} : float2_t{b[2 * e - 4], b[2 * e - 3]};
-    const bf16x2 h = __builtin_convertvector(x, bf16x2);
-    const float2_t r = x - __builtin_convertvector(h, float2_t);
-    const bf16x2 m = __builtin_convertvector(r, bf16x2);
-    const bf16x2 l = __builtin_convertvector(r - __builtin_convertvector(m, float2_t), bf16x2);
-    hi[2 * e] = h[0], hi[2 * e + 1] = h[1];
-    mid[2 * e] = m[0], mid[2 * e + 1] = m[1];
-    lo[2 * e] = l[0], lo[2 * e + 1] = l[1];
   }
 }
 

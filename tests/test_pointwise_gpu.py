@@ -409,3 +409,59 @@ def test_head_logits_match_f64(clef, H):
     # a chain of H / 64 adds and six butterfly steps: (H / 64 + 7) 2^-24 of the terms
     bound = (H / 64 + 8) * 2.0 ** -24 * (w.double().abs() @ x.double().abs())
     assert ((clef.head_logits(x, w).double() - ref).abs() <= bound).all()
+
+
+def _attention_f64(q, k, v, gate):
+    """q [heads, qn, d], k and v [kvh, kn, d], gate [qn, heads, d]."""
+    heads, qn, d = q.shape
+    kvh, kn, _ = k.shape
+    hidden = torch.ones((qn, kn), dtype=torch.bool, device="cuda").triu(kn - qn + 1)
+    y = torch.empty((qn, heads, d), dtype=torch.float64, device="cuda")
+    for h in range(heads):
+        s = q[h].double() @ k[h * kvh // heads].double().T / d ** 0.5
+        y[:, h] = torch.softmax(s.masked_fill(hidden, -torch.inf), -1) @ v[h * kvh // heads].double()
+    return (y * torch.sigmoid(gate.double())).reshape(qn, heads * d)
+
+
+@gpu
+@pytest.mark.parametrize("heads,kvh,d", [(4, 2, 256), (3, 1, 128), (2, 2, 64)])
+@pytest.mark.parametrize("qn,kn", [(1, 1), (1, 33), (15, 32), (16, 64), (65, 65), (64, 97), (100, 331), (130, 161)])
+def test_attention_f32_split_matches_f64(clef, heads, kvh, d, qn, kn):
+    """Tile edges of the f32 kernel (64 queries, two groups of 32-key tiles), values past kn
+    undefined, and gate and output rows without 16-byte alignment.  Scores up to ~6 carry a
+    rounding of 2^-24 relative through the exponential: 1e-5 of the largest value, 1e-6 in norm."""
+    gen = torch.Generator(device="cuda").manual_seed(71)
+    rnd = lambda *s: torch.randn(s, generator=gen, device="cuda")
+    q, k, v = rnd(heads, qn, d), rnd(kvh, kn, d), rnd(kvh, kn, d)
+    wide = rnd(qn, heads, 2 * d + 1)
+    vt = torch.full((kvh, d, max(64, (kn + 3) // 4 * 4)), float("nan"), device="cuda")
+    vt[:, :, :kn] = v.transpose(1, 2)
+    for gate in (wide[:, :, :d].contiguous(), wide[:, :, d + 1:]):
+        y = clef.attention_gated(q, k, vt, gate, kn=kn).double()
+        ref = _attention_f64(q, k, v, gate)
+        assert (y - ref).norm() <= 1e-6 * ref.norm()
+        assert (y - ref).abs().max() <= 1e-5 * v.abs().max()
+
+
+@gpu
+def test_attention_f32_values_the_split_does_not_hold(clef):
+    heads, kvh, qn, d = 2, 1, 150, 256
+    gen = torch.Generator(device="cuda").manual_seed(72)
+    rnd = lambda *s: torch.randn(s, generator=gen, device="cuda")
+    q, k, v, gate = rnd(heads, qn, d), rnd(kvh, qn, d), rnd(kvh, qn, d), rnd(qn, heads, d)
+    v[0, 0, 5], v[0, 0, 6] = float("inf"), -float("inf")  # key 0: every query sees it
+    v[0, :, 7] *= 1e-35
+    v[0, :, 8] = 0.0
+    q[1, 100] = float("nan")
+    vt = torch.zeros((kvh, d, 152), device="cuda")
+    vt[:, :, :qn] = v.transpose(1, 2)
+    y = clef.attention_gated(q, k, vt, gate, kn=qn).view(qn, heads, d)
+    ref = _attention_f64(q, k, v, gate).view(qn, heads, d)
+    bad = torch.zeros((qn, heads), dtype=torch.bool, device="cuda")
+    bad[100, 1] = True
+    assert torch.isnan(y[bad]).all()
+    y, ref = y[~bad], ref[~bad]
+    assert (y[:, 5] == float("inf")).all() and (y[:, 6] == -float("inf")).all()
+    assert (y[:, 7].double() - ref[:, 7]).norm() <= 1e-5 * ref[:, 7].norm()
+    assert (y[:, 8] == 0).all()
+    assert torch.allclose(y[:, 9:].double(), ref[:, 9:], rtol=1e-4, atol=1e-5)
