@@ -1121,31 +1121,60 @@ struct TileShape {
   int bm, bn;
   RingTile ring;
 };
-static TileShape gemm_f16_tile_shape(const GemmParams& p, int epilogue) {
-  const int n_eff = epilogue == 2 ? 2 * p.N : p.N;
+struct TileCost {
+  TileShape t;
+  double c;
+};
+static TileCost gemm_f16_tile_shape(int M, int N, int epilogue) {
+  const int n_eff = epilogue == 2 ? 2 * N : N;
   const long cus = device_cus();
   auto rounds = [&](int rows, int bn) {
-    const long tiles = (long)((p.M + rows - 1) / rows) * ((n_eff + bn - 1) / bn);
+    const long tiles = (long)((M + rows - 1) / rows) * ((n_eff + bn - 1) / bn);
     return (double)((tiles + cus - 1) / cus);
   };
   auto cost = [&](int rows, int bn, double per_out) { return rounds(rows, bn) * rows * bn * per_out; };
   auto paired = [&](int rows, int bn, double unit) { return (0.5 + 0.5 * rounds(rows, bn)) * unit; };
-  struct Cand {
-    TileShape t;
-    double c;
-  };
-  const Cand cands[] = {{{256, 256, kRingNone}, cost(256, 256, 1.0)},
-                        {{256, 192, kRingNone}, cost(256, 192, epilogue == 2 ? 1.22 : 1.1)},
-                        {{256, 128, kRingNone}, cost(256, 128, 1.2)},
-                        {{128, 128, kRingNone}, cost(128, 128, 1.5)},
-                        {{128, 64, kRing128x64}, rounds(128, 64) * 20000.0},
-                        {{64, 64, kRing64x64}, rounds(64, 64) * 14000.0},
-                        {{64, 32, kRing64x32}, paired(64, 32, 10200.0)},
-                        {{32, 16, kRing32x16}, epilogue == 2 ? 1e300 : paired(32, 16, 5900.0)}};
-  Cand best = cands[0];
-  for (const Cand& c : cands)
+  const TileCost cands[] = {{{256, 256, kRingNone}, cost(256, 256, 1.0)},
+                            {{256, 192, kRingNone}, cost(256, 192, epilogue == 2 ? 1.22 : 1.1)},
+                            {{256, 128, kRingNone}, cost(256, 128, 1.2)},
+                            {{128, 128, kRingNone}, cost(128, 128, 1.5)},
+                            {{128, 64, kRing128x64}, rounds(128, 64) * 20000.0},
+                            {{64, 64, kRing64x64}, rounds(64, 64) * 14000.0},
+                            {{64, 32, kRing64x32}, paired(64, 32, 10200.0)},
+                            {{32, 16, kRing32x16}, epilogue == 2 ? 1e300 : paired(32, 16, 5900.0)}};
+  TileCost best = cands[0];
+  for (const TileCost& c : cands)
     if (c.c < best.c) best = c;
-  return best.t;
+  return best;
+}
+
+// Rows of the first launch where two launches take less than one (else M):
+// whole rows of tiles up to a multiple of 256, the rest on the tile that suits
+// it.  A call of 256-row tiles a few rows past a whole number of rounds
+// otherwise pays a further round of large tiles that is nearly empty; a row
+// keeps its bits, as every tile shape sums in the same order.  The gap is the
+// second launch's start (2.9 us in the tiles' unit at K = 2048).  us, one
+// launch -> two, K = 2048: N = 12288 1290 rows 78.8 -> 67.0, 1400 78.3 -> 71.9,
+// 1500 79.8 -> 77.2; N = 9216 1800 rows 76.1 -> 68.9; SwiGLU N = 6144 1290
+// rows 85.1 -> 69.2, 2600 153 -> 124, 2800 154 -> 132.  A predicted gain below
+// 7% is not taken (it measured 0.98-1.02), nor is a call split that needs one
+// round of 256-row tiles, or smaller tiles (N = 2048, K = 6144, 2200 rows as
+// 2048 on 128 x 128 tiles and a rest: 67.9 -> 75.4).
+static int gemm_f16_split_rows(const GemmParams& p, int epilogue, const TileCost& one) {
+  int rows = p.M;
+  const int bn = epilogue == 2 ? one.t.bn / 2 : one.t.bn;
+  if (one.t.bm != 256 || (long)((p.M + 255) / 256) * ((p.N + bn - 1) / bn) <= device_cus()) return rows;
+  double best = 0.93 * one.c;
+  const double gap = 4000.0 * 2048 / p.K;
+  for (int j = 0; j < 3; ++j) {
+    const int m1 = (p.M / 256 - j) * 256;
+    if (m1 <= 0) break;
+    if (m1 == p.M) continue;
+    const double c =
+        gap + gemm_f16_tile_shape(m1, p.N, epilogue).c + gemm_f16_tile_shape(p.M - m1, p.N, epilogue).c;
+    if (c < best) best = c, rows = m1;
+  }
+  return rows;
 }
 
 template <int BM, int BN, int VM, int VN, int U, int S>
@@ -1161,8 +1190,7 @@ static int launch_ring(const GemmParams& p, int epilogue, hipStream_t s) {
   return check_launch("gemm");
 }
 
-int gemm_f16_dma_launch(const GemmParams& p, int epilogue, hipStream_t s) {
-  const TileShape t = gemm_f16_tile_shape(p, epilogue);
+static int launch_tiles(const GemmParams& p, int epilogue, const TileShape& t, hipStream_t s) {
   const int bn = t.bn;
   switch (t.ring) {
     case kRing32x16: return launch_ring<32, 16, 2, 1, 4, 3>(p, epilogue, s);
@@ -1181,6 +1209,19 @@ int gemm_f16_dma_launch(const GemmParams& p, int epilogue, hipStream_t s) {
   if (epilogue == 1)
     return bn == 256 ? launch<256, 256, 1>(p, s) : bn == 192 ? launch<256, 192, 1>(p, s) : launch<256, 128, 1>(p, s);
   return bn == 256 ? launch<256, 256, 2>(p, s) : bn == 192 ? launch<256, 192, 2>(p, s) : launch<256, 128, 2>(p, s);
+}
+
+int gemm_f16_dma_launch(const GemmParams& p, int epilogue, hipStream_t s) {
+  const TileCost one = gemm_f16_tile_shape(p.M, p.N, epilogue);
+  const int rows = gemm_f16_split_rows(p, epilogue, one);
+  if (rows == p.M) return launch_tiles(p, epilogue, one.t, s);
+  GemmParams a = p, b = p;
+  a.M = rows;
+  b.M = p.M - rows;
+  b.x = static_cast<const half_t*>(p.x) + (int64_t)rows * p.ldx;
+  b.y = static_cast<char*>(p.y) + (int64_t)rows * p.ldy * (epilogue != 1 && p.dtype_out == 1 ? 2 : 4);
+  if (int rc = launch_tiles(a, epilogue, gemm_f16_tile_shape(a.M, p.N, epilogue).t, s)) return rc;
+  return launch_tiles(b, epilogue, gemm_f16_tile_shape(b.M, p.N, epilogue).t, s);
 }
 
 }  // namespace clef

@@ -262,6 +262,32 @@ def test_gemm_small_tiles_write_only_their_rows(clef):
     assert (buf[M:] == 7).all() and (buf[:, :8] == 7).all() and (buf[:, 8 + N:] == 7).all()
 
 
+# a few rows past whole rounds of large tiles: one call as two launches (one
+# row, a partial small tile, most of a tile row; N off the tile edges)
+SPLIT_ROWS = [(1281, 12288, 2048), (1400, 12288, 1024), (1296, 12281, 1536), (1801, 9216, 2048), (2600, 6144, 2048)]
+
+
+@gpu
+@pytest.mark.parametrize("M,N,K", SPLIT_ROWS)
+def test_gemm_split_rows(clef, M, N, K):
+    """Every row equals the same row of calls of 700 and fewer rows, which are
+    single launches on other tiles; rows of a wider buffer, nothing else written."""
+    x, w = _inputs(24, M, N, K, torch.float16)
+    _, u = _inputs(25, 1, N, K, torch.float16)
+    parts = [slice(i, min(i + 700, M)) for i in range(0, M, 700)]
+    buf = torch.full((M + 2, N + 16), 7.0, device="cuda").half()
+    y = clef.gemm(x, w, out=buf[:M, 8:8 + N])
+    _check_f16(y, x, w)
+    assert torch.equal(y, torch.cat([clef.gemm(x[r], w) for r in parts]))
+    assert (buf[M:] == 7).all() and (buf[:, :8] == 7).all() and (buf[:, 8 + N:] == 7).all()
+    assert torch.equal(clef.gemm(x, w, out_dtype=torch.float32).half(), y)
+    h0 = torch.randn((M, N), device="cuda")
+    assert torch.equal(clef.gemm(x, w, residual=h0.clone(), out_dtype=torch.float16), h0 + y.float())
+    s = clef.gemm_swiglu(x, w, u)
+    assert torch.equal(s, clef.silu_mul(y.contiguous(), clef.gemm(x, u)))
+    assert torch.equal(s, torch.cat([clef.gemm_swiglu(x[r], w, u) for r in parts]))
+
+
 # f32 operands with 16-byte rows: each tile shape (32 x 32 .. 256 x 128), edges
 # and remainders in rows and columns, K of one float4, below one step, ragged
 # steps and stages
