@@ -215,6 +215,7 @@ extern "C" int clef_ragged_plan(const int32_t* cu_seqlens, int nseq, int T, int 
   if ((size_t)total > cap) return fail(-3, "ragged plan: the tables exceed their capacity");
   if (unit == 64) {
     for (int t = 0; t < kTabThreads; ++t) rg_scan_6(g, t, unit, ctab.data(), stab.data());
+    for (int c = 0; c < total; ++c) ctab[2 * c + 1] = chunk_tokens(ctab[2 * c + 1]);
   } else {
     for (int t = 0; t < kTabThreads; ++t) rg_attn_6(g, t, unit, total, ctab.data());
   }

@@ -30,9 +30,12 @@
 // factors (see the carry below).
 #pragma once
 #include "common.hpp"
+#include "ragged.hpp"
 #include "scan.hpp"
 
 namespace clef {
+
+int device_cus();  // of the current device (gemm_f16.hip)
 namespace {
 
 constexpr int kC = 64;   // chunk length
@@ -186,7 +189,7 @@ __device__ __forceinline__ bool chunk_span(const ScanParams& p, int c, int& t0, 
     if (c >= *p.nchunk_total) return false;
     const int2 e = p.chunk_tab[c];
     t0 = e.x;
-    n = e.y;
+    n = chunk_tokens(e.y);
   } else {
     t0 = c * kC;
     n = min(kC, p.T - t0);
@@ -647,9 +650,6 @@ __device__ __forceinline__ void lds_wait_all(const unsigned* flags, int n, unsig
 // these spans), so no table is read on the carry's paths; a lookup there
 // makes each step wait for it, and in-order vmcnt then drains every load
 // in flight behind it.
-struct CarryCtx;
-__device__ __forceinline__ void chunk_of(const CarryCtx& x, int c, int& t0, int& n);
-
 struct CarryCtx {
   int h, hk, j0, jc;
   bool col_ok;
@@ -661,9 +661,26 @@ struct CarryCtx {
   float* fin;         // its final state or null
 };
 
-__device__ __forceinline__ void chunk_of(const CarryCtx& x, int c, int& t0, int& n) {
-  t0 = x.t0s + c * kC;
-  n = min(kC, x.lens - c * kC);
+// The chunk table's entry c, through the scalar cache: a vector load would sit
+// among the prefetches that the waves count.  (The table is written by an
+// earlier kernel.)
+typedef const __attribute__((address_space(4))) int const_int;
+__device__ __forceinline__ int2 chunk_entry(const ScanParams& p, int c) {
+  const_int* e = (const_int*)reinterpret_cast<uintptr_t>(p.chunk_tab) + 2 * __builtin_amdgcn_readfirstlane(c);
+  return int2{e[0], e[1]};
+}
+
+// VL 0: one sequence, 1: one sequence of a ragged batch, 2: all of them in a row
+template <int VL>
+__device__ __forceinline__ void chunk_of(const ScanParams& p, const CarryCtx& x, int c, int& t0, int& n) {
+  if constexpr (VL == 2) {
+    const int2 e = chunk_entry(p, c);
+    t0 = e.x;
+    n = chunk_tokens(e.y);
+  } else {
+    t0 = x.t0s + c * kC;
+    n = min(kC, x.lens - c * kC);
+  }
 }
 
 // EPF elements k.. of raw key row r in a slot's key region, as a CT fragment.
@@ -730,11 +747,11 @@ __device__ __forceinline__ typename Mma<CT>::frag query_frag(const IT* row, int 
 // The raw key rows of chunk c element by element, for rows that are not
 // whole 16-byte vectors (dk < DK or unaligned rows): stored in the layout the
 // key DMA produces (below), with zeros past dk.
-template <class CT, class IT, int DK, bool VL>
+template <class CT, class IT, int DK, int VL>
 __device__ __forceinline__ void carry_keys_slow(const ScanParams& p, const CarryCtx& x, char* keys, int c) {
   typedef Carry<CT, IT, DK> K;
   int t0, n;
-  chunk_of(x, c, t0, n);
+  chunk_of<VL>(p, x, c, t0, n);
   const char* base = reinterpret_cast<const char*>(static_cast<const IT*>(p.k) + (int64_t)t0 * p.sqk +
                                                    (int64_t)x.hk * p.dk);
   const int64_t rowb = p.sqk * (int64_t)sizeof(IT);
@@ -760,7 +777,7 @@ __device__ __forceinline__ void carry_keys_slow(const ScanParams& p, const Carry
 // instead: chunk i + 1 + PREF during chunk i (the recurrence reads chunk
 // i + 1's keys during chunk i when it prefetches), so they are published by
 // the barrier that ends chunk i - PREF.
-template <class CT, class IT, int DK, bool VL, int LW, bool FAST>
+template <class CT, class IT, int DK, int VL, int LW, bool FAST>
 __device__ __forceinline__ void carry_loader_w(const ScanParams& p, const CarryCtx& x, char* ring) {
   typedef Carry<CT, IT, DK> K;
   constexpr int NDK = K::NDK, NU = K::G::NBU;
@@ -773,10 +790,10 @@ __device__ __forceinline__ void carry_loader_w(const ScanParams& p, const CarryC
   auto slot = [&](int c) { return ring + (c % K::D0) * K::SLOT; };
   auto issue = [&](int c) {
     char* s = slot(c);
-    const int64_t cg = (VL ? x.c0 : 0) + c;
+    const int64_t cg = (VL == 1 ? x.c0 : 0) + c;
     if constexpr (FAST && KQ1 > KQ0) {
       int t0, n;
-      chunk_of(x, c, t0, n);
+      chunk_of<VL>(p, x, c, t0, n);
       const char* base = reinterpret_cast<const char*>(static_cast<const IT*>(p.k) + (int64_t)t0 * p.sqk +
                                                        (int64_t)x.hk * p.dk);
       const int64_t rowb = p.sqk * (int64_t)sizeof(IT);
@@ -821,7 +838,7 @@ __device__ __forceinline__ void carry_loader_w(const ScanParams& p, const CarryC
   lds_barrier();  // outputs of the last chunk
 }
 
-template <class CT, class IT, int DK, bool VL, int LW>
+template <class CT, class IT, int DK, int VL, int LW>
 __device__ __forceinline__ void carry_loader_fs(const ScanParams& p, const CarryCtx& x, char* ring) {
   if (p.vec_qk && p.dk == DK)
     carry_loader_w<CT, IT, DK, VL, LW, true>(p, x, ring);
@@ -829,7 +846,7 @@ __device__ __forceinline__ void carry_loader_fs(const ScanParams& p, const Carry
     carry_loader_w<CT, IT, DK, VL, LW, false>(p, x, ring);
 }
 
-template <class CT, class IT, int DK, bool VL>
+template <class CT, class IT, int DK, int VL>
 __device__ __forceinline__ void carry_loader(const ScanParams& p, const CarryCtx& x, int lw, char* ring) {
   typedef Carry<CT, IT, DK> K;
   static_assert(K::NLOAD >= 1 && K::NLOAD <= 3, "one to three loader waves");
@@ -851,7 +868,7 @@ __device__ __forceinline__ void carry_loader(const ScanParams& p, const CarryCtx
 //   S_R <- e^gam_last S_R + U_R Y (the wave's rows of U).
 // With one wave this is Y = V - (a e^gam) K S.  S_i and Y_i go to the output
 // waves through `hand`.
-template <class CT, class IT, int DK, bool VL, bool CAP, int R>
+template <class CT, class IT, int DK, int VL, bool CAP, int R>
 __device__ __forceinline__ void carry_recurrence(const ScanParams& p, const CarryCtx& x, const char* ring,
                                                  typename Mma<CT>::frag* hand, float4_t* xch, unsigned* xflag) {
   typedef Carry<CT, IT, DK> K;
@@ -861,19 +878,41 @@ __device__ __forceinline__ void carry_recurrence(const ScanParams& p, const Carr
   constexpr int NREC = K::NREC, KPR = K::KPR, SPR = K::SPR, KB0 = R * KPR, S0 = R * SPR;
   const int lane = x.lane, grp = x.grp, col = x.col;
   const int dk = p.dk, dv = p.dv;
-  const float* init = VL ? x.init : p.initial;
-  float* fin = VL ? x.fin : p.final_state;
+  const float* init = VL == 1 ? x.init : p.initial;
+  float* fin = VL == 1 ? x.fin : p.final_state;
 
   float4_t S[SPR];
+  // a head's state through a buffer of its dk x dv floats (no state: of none):
+  // rows past dk and columns past dv (their lanes add 2^31) fall outside
+  const uint32_t slane = (uint32_t)x.jc * 4u + (x.col_ok ? 0u : 0x80000000u);
+  auto state_off = [&](int s, int i) {
+    return (int)((uint32_t)slot_index<CT>(S0 + s, 4 * grp + i) * (uint32_t)dv * 4u + slane);
+  };
+  const int64_t shead = (int64_t)x.h * dk * dv;
+  auto load_state = [&](const float* from) {
+    const __amdgpu_buffer_rsrc_t r = make_rsrc(from ? from + shead : nullptr, from ? dk * dv * 4 : 0);
 #pragma unroll
-  for (int s = 0; s < SPR; ++s)
+    for (int s = 0; s < SPR; ++s)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = slot_index<CT>(S0 + s, 4 * grp + i);
-      float v = 0.0f;
-      if (init && row < dk && x.col_ok) v = init[((int64_t)x.h * dk + row) * dv + x.jc];
-      S[s][i] = v;
-    }
+      for (int i = 0; i < 4; ++i) S[s][i] = bits_value<float>(buffer_load_bits<float>(r, state_off(s, i)));
+  };
+  auto store_state = [&](float* to) {
+    const __amdgpu_buffer_rsrc_t r = make_rsrc(to + shead, dk * dv * 4);
+#pragma unroll
+    for (int s = 0; s < SPR; ++s)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) buffer_store(r, state_off(s, j), S[s][j], 0.0f);
+  };
+  const int64_t fin_stride = (int64_t)p.Hv * dk * dv;
+  // VL 2: the table entries of this chunk, the next and the one after
+  int2 e0 = {0, 0}, e1 = e0, e2 = e0;
+  if constexpr (VL == 2) {
+    e0 = chunk_entry(p, 0);
+    e1 = chunk_entry(p, min(1, x.nchunks - 1));
+    load_state(init ? init + chunk_seq(e0.y) * p.init_stride : nullptr);
+  } else {
+    load_state(init);
+  }
   frag Sf[KPR];
 #pragma unroll
   for (int k = 0; k < KPR; ++k) Sf[k] = pack_frag(S, k, CT(0));
@@ -887,9 +926,14 @@ __device__ __forceinline__ void carry_recurrence(const ScanParams& p, const Carr
   const IT* vbase = static_cast<const IT*>(p.v) + (int64_t)x.h * dv + x.j0;
   const uint32_t vlane = (uint32_t)col * (uint32_t)sizeof(IT) + (x.col_ok ? 0u : 0x80000000u);
   const uint32_t vrow = (uint32_t)p.sv * (uint32_t)sizeof(IT);
-  auto load_v = [&](uint32_t* vb, int c) {
+  auto load_v = [&](uint32_t* vb, int c, const int2& e) {
     int t0, n;
-    chunk_of(x, min(c, x.nchunks - 1), t0, n);
+    if constexpr (VL == 2) {
+      t0 = e.x;
+      n = chunk_tokens(e.y);
+    } else {
+      chunk_of<VL>(p, x, min(c, x.nchunks - 1), t0, n);
+    }
     const __amdgpu_buffer_rsrc_t r = make_rsrc(vbase + (int64_t)t0 * p.sv, n * (int)p.sv * (int)sizeof(IT));
 #pragma unroll
     for (int t = 0; t < 4; ++t)
@@ -900,8 +944,8 @@ __device__ __forceinline__ void carry_recurrence(const ScanParams& p, const Carr
   constexpr int NV = R == 0 ? 16 : 1;
   uint32_t va[NV], vb[NV];
   if constexpr (R == 0) {
-    load_v(va, 0);
-    load_v(vb, 1);
+    load_v(va, 0, e0);
+    load_v(vb, 1, e1);
   }
   // this lane's key rows (slot order) and k offset within each k-block
   int krow[4];
@@ -923,6 +967,7 @@ __device__ __forceinline__ void carry_recurrence(const ScanParams& p, const Carr
     const frag* uslot = reinterpret_cast<const frag*>(slot + K::UOFF);
     const float* scs = reinterpret_cast<const float*>(slot + K::SOFF);  // a e^gam, b e^gam, gam, e^gam
     frag* hs = hand + (i & 1) * (NKX + NKT) * 64;
+    if constexpr (VL == 2) e2 = chunk_entry(p, min(i + 2, x.nchunks - 1));
     // the chunk's keys: read during the previous chunk, or up front
     if constexpr (!K::PREF) load_k(i);
     float4_t ya[4], X[4];
@@ -950,6 +995,12 @@ __device__ __forceinline__ void carry_recurrence(const ScanParams& p, const Carr
     for (int k = 0; k < KPR; ++k) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) Mma<CT>::mma(X[t], kf[t][k], Sf[k]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (VL == 2) {
+      // scalar loads return out of order with LDS reads: taken here, where
+      // only row factors are outstanding, not among the U reads
+      asm volatile("" ::"s"(e2.x), "s"(e2.y));
       __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (EARLY_U) {
@@ -1038,9 +1089,20 @@ __device__ __forceinline__ void carry_recurrence(const ScanParams& p, const Carr
       __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (K::PREF) load_k(i + 1);
+    if constexpr (VL == 2) {
+      // a sequence ends: its state out, the next one's in
+      if (chunk_last(e0.y)) {
+        if (fin) store_state(fin + chunk_seq(e0.y) * fin_stride);
+        load_state(init ? init + chunk_seq(e1.y) * p.init_stride : nullptr);
+        // waited for in here, or every chunk would wait where the paths join
+#pragma unroll
+        for (int s = 0; s < SPR; ++s) asm volatile("" : "+v"(S[s]));
+      }
+    }
 #pragma unroll
     for (int k = 0; k < KPR; ++k) Sf[k] = pack_frag(S, k, CT(0));
-    if constexpr (R == 0) load_v(vbuf, i + 2);
+    if constexpr (R == 0) load_v(vbuf, i + 2, e2);
+    if constexpr (VL == 2) e0 = e1, e1 = e2;
     lds_barrier();  // end of chunk i
   };
   int i = 0;
@@ -1051,21 +1113,14 @@ __device__ __forceinline__ void carry_recurrence(const ScanParams& p, const Carr
   if (i < x.nchunks) step(i, va);
   lds_barrier();  // outputs of the last chunk
 
-  if (fin) {
-#pragma unroll
-    for (int s = 0; s < SPR; ++s)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int row = slot_index<CT>(S0 + s, 4 * grp + j);
-        if (row < dk && x.col_ok) fin[((int64_t)x.h * dk + row) * dv + x.jc] = S[s][j];
-      }
-  }
+  if constexpr (VL != 2)
+    if (fin) store_state(fin);
 }
 
 // Output waves: O of chunk c during chunk c+1, TPW tiles of 16 rows (token
 // order) from row 16 TPW ow: O = diag(b e^gam) (Q S) + N Y.  Query rows, N
 // blocks and the row factors are loaded into registers OD chunks ahead.
-template <class CT, class IT, int DK, class OT, bool VL, bool VEC>
+template <class CT, class IT, int DK, class OT, int VL, bool VEC>
 __device__ __forceinline__ void carry_outputs(const ScanParams& p, const CarryCtx& x, int ow,
                                               const typename Mma<CT>::frag* hand) {
   typedef Carry<CT, IT, DK> K;
@@ -1081,8 +1136,8 @@ __device__ __forceinline__ void carry_outputs(const ScanParams& p, const CarryCt
   auto load_o = [&](Ops& o, int c) {
     const int cc = min(c, x.nchunks - 1);
     int t0, n;
-    chunk_of(x, cc, t0, n);
-    const int64_t cg = (VL ? x.c0 : 0) + cc;
+    chunk_of<VL>(p, x, cc, t0, n);
+    const int64_t cg = (VL == 1 ? x.c0 : 0) + cc;
     const frag* nf = static_cast<const frag*>(p.Nf) + (cg * p.Hv + x.h) * G::NBN * 64 + lane;
     const float* scs = p.sc + (cg * p.Hv + x.h) * 256;
 #pragma unroll
@@ -1114,7 +1169,7 @@ __device__ __forceinline__ void carry_outputs(const ScanParams& p, const CarryCt
 #pragma unroll
     for (int b = 0; b < NKT; ++b) yf[b] = hs[(NKX + b) * 64 + lane];
     int t0, n;
-    chunk_of(x, c, t0, n);
+    chunk_of<VL>(p, x, c, t0, n);
     // rows past the end of the sequence fall outside the buffer range: dropped
     const __amdgpu_buffer_rsrc_t r = make_rsrc(out + (int64_t)t0 * p.so, n * (int)p.so * (int)sizeof(OT));
 #pragma unroll
@@ -1143,11 +1198,22 @@ __device__ __forceinline__ void carry_outputs(const ScanParams& p, const CarryCt
     if (c + d < x.nchunks) ostep(c + d, ops[d]);
 }
 
-// MODE 0: one sequence; 1: one sequence with a captured state; 2: a ragged batch.
+// MODE 0: one sequence; 1: one sequence with a captured state; 2: a ragged
+// batch, a work-group per sequence; 3: a ragged batch, a work-group walks all
+// sequences' chunks in token order.
+// Bound: the recurrence's serial chain, about 1 us a chunk (f16, dk 128).  One
+// work-group fills a CU's LDS, so with 256 or more (head, columns) the batch's
+// sequences take turns on a CU, and in MODE 2 each turn starts with an empty
+// ring and register pipeline, about 5 us.  MODE 3 keeps both full across the
+// boundaries (a boundary costs 0.7 us, the states out and in).  32 heads x 128,
+// us: 8 sequences of 64-1200 tokens, 5003 in all, f16 119 -> 85, f32 423 -> 385;
+// 16 of 12 tokens 90 -> 24, 168 -> 89; 64 of 64 tokens 372 -> 114, 743 -> 340;
+// 1200 + 800 tokens 43 -> 36, 160 -> 157.
 template <class CT, class IT, int DK, int MODE>
 __global__ __launch_bounds__((Carry<CT, IT, DK>::THREADS)) void scan_carry(ScanParams p) {
   typedef Carry<CT, IT, DK> K;
-  constexpr bool VL = MODE == 2, CAP = MODE == 1;
+  constexpr int VL = MODE == 2 ? 1 : MODE == 3 ? 2 : 0;
+  constexpr bool CAP = MODE == 1;
   __shared__ __attribute__((aligned(1024))) char ring[K::D0 * K::SLOT];
   __shared__ __attribute__((aligned(16))) typename K::frag hand[2 * (K::G::NKX + K::G::NKT) * 64];
   __shared__ __attribute__((aligned(16))) float4_t xch[K::NREC > 1 ? K::NREC * 4 * 64 : 1];
@@ -1168,9 +1234,9 @@ __global__ __launch_bounds__((Carry<CT, IT, DK>::THREADS)) void scan_carry(ScanP
   const int ntiles = (p.dv + kVT - 1) / kVT;
   const int per_seq = p.Hv * ntiles;
   int L = blockIdx.x;
-  if (!VL && (nwg & 7) == 0) {
+  if (VL != 1 && (nwg & 7) == 0) {
     L = (blockIdx.x & 7) * (nwg >> 3) + (blockIdx.x >> 3);
-  } else if (VL && (per_seq & 7) == 0) {
+  } else if (VL == 1 && (per_seq & 7) == 0) {
     const int b = L % per_seq;
     L += (b & 7) * (per_seq >> 3) + (b >> 3) - b;
   }
@@ -1180,7 +1246,8 @@ __global__ __launch_bounds__((Carry<CT, IT, DK>::THREADS)) void scan_carry(ScanP
   int seq = 0;
   x.c0 = 0;
   x.nchunks = p.nchunks;
-  if (VL) {
+  if (VL == 2) x.nchunks = *p.nchunk_total;
+  if (VL == 1) {
     const int4 e = p.seq_tab[slot];
     seq = e.x;
     x.c0 = e.y;
@@ -1196,7 +1263,25 @@ __global__ __launch_bounds__((Carry<CT, IT, DK>::THREADS)) void scan_carry(ScanP
   x.cap_chunk = p.capture > 0 ? (p.capture - 1) / kC : -1;
   x.cap_row = p.capture > 0 ? (p.capture - 1) % kC : 0;
 
-  if (VL && x.nchunks == 0) {  // empty sequence: the final state is the initial one
+  if (VL == 2) {  // empty sequences: the final state is the initial one
+    if (wave == 0 && p.final_state)
+      for (int s0 = 0; s0 < p.nseq; s0 += 64) {
+        const int sq = min(s0 + x.lane, p.nseq - 1);
+        uint64_t empty = __ballot(s0 + x.lane < p.nseq && p.cu_seqlens[sq] == p.cu_seqlens[sq + 1]);
+        for (; empty; empty &= empty - 1) {
+          const int e = s0 + __builtin_ctzll(empty);
+          const float* from = p.initial ? p.initial + e * p.init_stride : nullptr;
+          float* to = p.final_state + (int64_t)e * p.Hv * p.dk * p.dv;
+          if (x.col_ok)
+            for (int r = x.grp; r < p.dk; r += 4) {
+              const int64_t o = ((int64_t)x.h * p.dk + r) * p.dv + x.jc;
+              to[o] = from ? from[o] : 0.0f;
+            }
+        }
+      }
+    if (x.nchunks == 0) return;
+  }
+  if (VL == 1 && x.nchunks == 0) {  // empty sequence: the final state is the initial one
     if (wave == 0 && x.fin && x.col_ok)
       for (int r = x.grp; r < p.dk; r += 4) {
         const int64_t o = ((int64_t)x.h * p.dk + r) * p.dv + x.jc;
@@ -1206,10 +1291,10 @@ __global__ __launch_bounds__((Carry<CT, IT, DK>::THREADS)) void scan_carry(ScanP
   }
   x.t0s = 0;
   x.lens = p.T;
-  if (VL) {  // the first and last chunk of the sequence
+  if (VL == 1) {  // the first and last chunk of the sequence
     const int2 a = p.chunk_tab[x.c0], z = p.chunk_tab[x.c0 + x.nchunks - 1];
     x.t0s = a.x;
-    x.lens = z.x + z.y - a.x;
+    x.lens = z.x + chunk_tokens(z.y) - a.x;
   }
   if (wave < K::NREC) {
     if (wave == 0) carry_recurrence<CT, IT, DK, VL, CAP, 0>(p, x, ring, hand, xch, xflag);
@@ -1253,7 +1338,11 @@ int launch_dk(const ScanParams& p, hipStream_t stream) {
   const int ntiles = (p.dv + kVT - 1) / kVT;
   const int nseq = p.seq_tab ? p.nseq : 1;
   const dim3 block(Carry<CT, IT, DK>::THREADS);
-  if (p.seq_tab)
+  // a batch walks in a row where its (head, columns) fill the CUs; with fewer,
+  // sequences side by side use the idle ones
+  if (p.seq_tab && p.Hv * ntiles >= device_cus())
+    hipLaunchKernelGGL((scan_carry<CT, IT, DK, 3>), dim3(p.Hv * ntiles), block, 0, stream, p);
+  else if (p.seq_tab)
     hipLaunchKernelGGL((scan_carry<CT, IT, DK, 2>), dim3(nseq * p.Hv * ntiles), block, 0, stream, p);
   else if (p.capture > 0)
     hipLaunchKernelGGL((scan_carry<CT, IT, DK, 1>), dim3(p.Hv * ntiles), block, 0, stream, p);

@@ -89,8 +89,14 @@ __host__ __device__ inline void rg_count_5(const Ragged& g, int tid, int* total)
   *total = acc;
 }
 
-// Scan, step 6: per sequence its chunks' token spans (ctab: first token,
-// tokens) and its entry in stab ({sequence, first chunk, chunks, 0}) at its
+// A scan chunk's second table word: tokens (1..64), whether it is the last of
+// its sequence, the sequence.
+__host__ __device__ inline int chunk_word(int tokens, bool last, int seq) { return tokens | (int)last << 7 | seq << 8; }
+__host__ __device__ inline int chunk_tokens(int w) { return w & 127; }
+__host__ __device__ inline bool chunk_last(int w) { return (w >> 7 & 1) != 0; }
+__host__ __device__ inline int chunk_seq(int w) { return w >> 8; }
+
+// Scan, step 6: per sequence its chunks (ctab: first token, chunk_word) and its entry in stab ({sequence, first chunk, chunks, 0}) at its
 // rank by chunk count (most first, ties in sequence order).
 __host__ __device__ inline void rg_scan_6(const Ragged& g, int tid, int chunk, int* ctab, int* stab) {
   int s0, s1;
@@ -108,7 +114,7 @@ __host__ __device__ inline void rg_scan_6(const Ragged& g, int tid, int chunk, i
     const int t0 = g.R[s], len = g.R[s + 1] - t0;
     for (int c = 0; c < nc; ++c) {
       ctab[2 * (first + c)] = t0 + c * chunk;
-      ctab[2 * (first + c) + 1] = rg_min(chunk, len - c * chunk);
+      ctab[2 * (first + c) + 1] = chunk_word(rg_min(chunk, len - c * chunk), c == nc - 1, s);
     }
     first += nc;
   }

@@ -261,3 +261,32 @@ def test_short_scan_prepared_per_v_head_equals_long_scan(clef, precision, T):
     if T % 64 == 0:
         _, captured, _ = scan.prefill(*x, capture=T)
         assert torch.equal(final, captured)
+
+
+@gpu
+@pytest.mark.parametrize("precision,dtype,dk", [("mixed", torch.float16, 128), ("strict", torch.float32, 128),
+                                                ("mixed", torch.float32, 100), ("strict", torch.float16, 64),
+                                                ("strict", torch.float32, 32)])
+@pytest.mark.parametrize("initial", ["none", "shared", "each"])
+@pytest.mark.parametrize("lens", [[0, 1, 64, 65, 0, 130, 7, 63, 192, 0], [0, 0], [300], [1] * 70])
+def test_scan_varlen_walked_in_a_row_equals_single_scans(clef, precision, dtype, dk, initial, lens):
+    """Ragged batches with enough heads and columns to fill the GPU walk all
+    sequences in one work-group per (head, columns): each equals the same
+    sequence scanned alone, bit for bit; an empty one (first, last, repeated,
+    all of them) hands its initial state through."""
+    Hk, Hv, dv, nseq, T = 16, 32, 128, len(lens), max(sum(lens), 1)
+    x = case_inputs(15, T, Hk, Hv, dk, dv, dtype=dtype)
+    cu = torch.tensor(np.concatenate([[0], np.cumsum(lens)]), dtype=torch.int32, device="cuda")
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    shape = (Hv, dk, dv) if initial == "shared" else (nseq, Hv, dk, dv)
+    init = None if initial == "none" else 0.1 * torch.randn(shape, generator=gen, device="cuda")
+    scan = clef.DeltaScan(dk, dv, precision)
+    out, final = scan.prefill_varlen(*x, cu, initial=init)
+    for s, (a, b) in enumerate(zip(cu[:-1].tolist(), cu[1:].tolist())):
+        s0 = init if initial != "each" else init[s]
+        if a == b:
+            assert torch.equal(final[s], torch.zeros_like(final[s]) if s0 is None else s0)
+            continue
+        o, _, f = scan.prefill(*(t[a:b] for t in x), initial=s0)
+        assert torch.equal(out[a:b], o)
+        assert torch.equal(final[s], f)
