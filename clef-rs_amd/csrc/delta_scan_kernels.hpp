@@ -139,6 +139,22 @@ __device__ __forceinline__ float bits_to_f32(uint32_t b, int dtype) {
 // full precision; results below the normal range may flush to zero.
 __device__ __forceinline__ float decay_exp(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504088896341f); }
 
+// Inclusive running sum over the 64 lanes by DPP moves: within rows of 16
+// (shifts by 1, 2, 4, 8, zeros in), then each row's total into the rows after it.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_or_zero(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xf, false));
+}
+__device__ __forceinline__ float wave_running_sum(float v) {
+  v += dpp_or_zero<0x111, 0xf>(v);  // row_shr:1
+  v += dpp_or_zero<0x112, 0xf>(v);  // row_shr:2
+  v += dpp_or_zero<0x114, 0xf>(v);  // row_shr:4
+  v += dpp_or_zero<0x118, 0xf>(v);  // row_shr:8
+  v += dpp_or_zero<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+  v += dpp_or_zero<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+  return v;
+}
+
 __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
 
 // s_waitcnt vmcnt(N) (gfx9 encoding: vmcnt in bits 3:0 and 15:14).
@@ -232,6 +248,15 @@ __device__ __forceinline__ float l2norm_row(const float* x, float extra, CT* dst
 // ---------------------------------------------------------------------------
 constexpr int kPW = 8;  // waves of a scan_prepare work-group
 
+// Bound: the chain of a v-head's steps (decay, A and M, the inverse's diagonal
+// and off-diagonal blocks, U, N), each a few LDS round trips long with most
+// waves idle; at T = 4096 two work-groups of two heads run twice on each CU.
+// The next head's decay beside this one's inversion, a tile position's A and M
+// on one wave, reads of the inversion requested ahead and its off-diagonal
+// blocks without barriers took 12100 of 31800 cycles to 7500 of 27000 (f16).
+// 16 / 32 heads x 128, us, f16 and f32: T = 4096 37.5 -> 33.8, 88.7 -> 82.3;
+// T = 1000 18.0 -> 16.2, 24.6 -> 22.8; T = 100 10.8 -> 8.8, 15.3 -> 14.4.
+//
 // Two work-groups per CU (16 waves, 128 registers each) where the LDS holds
 // two; f32 products with 128-wide keys need more LDS than half a CU.
 template <class CT, class IT, int DK>
@@ -255,10 +280,11 @@ __global__ __launch_bounds__(64 * kPW, (sizeof(CT) == 4 && DK > 64) ? 2 : 4) voi
   constexpr int kBytesR = kBytesKQ > kBytes3 ? kBytesKQ : kBytes3;
   __shared__ __attribute__((aligned(16))) CT sKT[DK * LDT];  // K^ transposed [e][token]
   __shared__ __attribute__((aligned(16))) char sR[kBytesR];
-  __shared__ __attribute__((aligned(16))) float sGam[kC];
-  __shared__ __attribute__((aligned(16))) float sBeta[kC];
-  __shared__ __attribute__((aligned(16))) float sW[kC];   // exp(gam_last - gam)
-  __shared__ __attribute__((aligned(16))) float sWc[kC];  // capture weights
+  // row factors of a v-head, and of the next one (double-buffered)
+  __shared__ __attribute__((aligned(16))) float sGam2[2][kC];
+  __shared__ __attribute__((aligned(16))) float sBeta2[2][kC];
+  __shared__ __attribute__((aligned(16))) float sW2[2][kC];   // exp(gam_last - gam)
+  __shared__ __attribute__((aligned(16))) float sWc2[2][kC];  // capture weights
   __shared__ __attribute__((aligned(16))) float sInv[2][kC];  // row factors: keys 1/|k|, queries qscale/|q|
   CT* sK = reinterpret_cast<CT*>(sR);
   CT* sQ = sK + kC * LDR;
@@ -280,7 +306,7 @@ __global__ __launch_bounds__(64 * kPW, (sizeof(CT) == 4 && DK > 64) ? 2 : 4) voi
 
   // ---- 1. loads: q/k rows (clamped), g and beta of the first v-head
   uint32_t gbits = 0, bbits = 0;
-  if (wave == 0) {
+  if (wave == kPW - 1) {
     const int64_t gi = (int64_t)(t0 + min(lane, n - 1)) * p.sgb + (int64_t)hk * rep + v0;
     gbits = load_bits(p.g, gi, p.dtype_gb);
     bbits = load_bits(p.beta, gi, p.dtype_gb);
@@ -323,25 +349,57 @@ __global__ __launch_bounds__(64 * kPW, (sizeof(CT) == 4 && DK > 64) ? 2 : 4) voi
     for (int j = 0; j < EPF; ++j) f[j] = sK[(tok0 + j) * LDR + e];
     *reinterpret_cast<frag*>(sKT + e * LDT + tok0) = f;
   }
-  // 20 lower 16x16 tiles: K^K^T (jobs 0-9) and Q^K^T (jobs 10-19); wave w
-  // takes the jobs w, w + kPW, ...
-  constexpr int JPW = (20 + kPW - 1) / kPW;
-  float4_t gram[JPW];
-#pragma unroll
-  for (int s = 0; s < JPW; ++s) {
-    const int job = wave + kPW * s;
-    if (job >= 20) break;
-    const bool isqk = job >= 10;
-    const int idx = isqk ? job - 10 : job;
-    const int tr = idx >= 6 ? 3 : idx >= 3 ? 2 : idx >= 1 ? 1 : 0;
-    const int tc = idx - tr * (tr + 1) / 2;
+  // The 10 lower 16x16 tile positions, each K^K^T and Q^K^T: wave w holds both
+  // tiles of position w (they share the decay ratios of 3b) and the four tiles
+  // of positions 8 and 9 go to waves 3..6 one by one.
+  auto tile_row = [](int idx) { return idx >= 6 ? 3 : idx >= 3 ? 2 : idx >= 1 ? 1 : 0; };
+  auto gram_tile = [&](bool isqk, int idx) {
+    const int tr = tile_row(idx), tc = idx - tr * (tr + 1) / 2;
     const CT* a_src = (isqk ? sQ : sK) + (16 * tr + col) * LDR + grp * EPF;
     const CT* b_src = sK + (16 * tc + col) * LDR + grp * EPF;
     float4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kb = 0; kb < NKX; ++kb) Mma<CT>::mma(acc, load_frag<CT>(a_src + kb * KB), load_frag<CT>(b_src + kb * KB));
-    gram[s] = acc;
-  }
+    return acc;
+  };
+  const bool extra = wave >= 3 && wave < 7, xkk = wave & 1;  // waves 3, 5: K^K^T, 4, 6: Q^K^T
+  const int xidx = 8 + ((wave - 3) >> 1);
+  const float4_t gkk = gram_tile(false, wave), gqk = gram_tile(true, wave);
+  float4_t gx = {0.f, 0.f, 0.f, 0.f};
+  if (extra) gx = gram_tile(!xkk, xidx);
+
+  // Cumulative decay and the per-row factors of v-head v, by one wave (lane =
+  // token): the carry's row factors 1/|k| e^gam (for V - e^gam K^ S) and
+  // qscale/|q| e^gam (for e^gam Q^ S), gam (capture) and e^gam.  The first
+  // v-head's here, the next one's while wave 0 inverts a head's diagonal
+  // blocks; the running sum moves by DPP (six shuffles through LDS took as
+  // long as that inversion).
+  auto head_rows = [&](int v) {
+    const int h = hk * rep + v, buf = (v - v0) & 1;
+    const float gv = lane < n ? bits_to_f32(gbits, p.dtype_gb) : 0.0f;
+    const float bv = lane < n ? bits_to_f32(bbits, p.dtype_gb) : 0.0f;
+    if (v + 1 < v1) {  // the next v-head's g and beta, awaited a head later
+      const int64_t gi = (int64_t)(t0 + min(lane, n - 1)) * p.sgb + h + 1;
+      gbits = load_bits(p.g, gi, p.dtype_gb);
+      bbits = load_bits(p.beta, gi, p.dtype_gb);
+    }
+    const float cs = wave_running_sum(gv);
+    const float gl = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cs), kC - 1));
+    sGam2[buf][lane] = cs;
+    sBeta2[buf][lane] = bv;
+    sW2[buf][lane] = decay_exp(gl - cs);
+    if (chunk == cap_chunk) {
+      const float gcap = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cs), cap_row));
+      sWc2[buf][lane] = lane <= cap_row ? decay_exp(gcap - cs) : 0.0f;
+    }
+    const float eg = decay_exp(cs);
+    float* sc = p.sc + ((int64_t)chunk * p.Hv + h) * 256;
+    sc[lane] = sInv[0][lane] * eg;
+    sc[64 + lane] = sInv[1][lane] * eg;
+    sc[128 + lane] = cs;
+    sc[192 + lane] = eg;
+  };
+  if (wave == kPW - 1) head_rows(v0);
   lds_barrier();  // sK / sQ are dead from here on
   // zeros that no v-head rewrites: the six 16x16 blocks of sTT below its
   // diagonal blocks (Tm above them) and the six tiles of sM above its diagonal
@@ -354,66 +412,56 @@ __global__ __launch_bounds__(64 * kPW, (sizeof(CT) == 4 && DK > 64) ? 2 : 4) voi
   }
 
   // ---- 3. per v-head
+  const int lane_of_wave = lane;
   for (int v = v0; v < v1; ++v) {
+    // the lane's addresses are formed anew for each head: kept from one to the
+    // next they spilled
+    int lane = lane_of_wave;
+    asm volatile("" : "+v"(lane));
+    const int col = lane & 15, grp = lane >> 4;
     const int h = hk * rep + v;
-    uint32_t gnext = 0, bnext = 0;
     const int64_t cv = (int64_t)chunk * p.Hv + h;
-    // 3a. cumulative decay and the per-row factors (wave 0, lane = token):
-    //     the carry's row factors 1/|k| e^gam (for V - e^gam K^ S) and
-    //     qscale/|q| e^gam (for e^gam Q^ S), gam (capture) and e^gam
-    if (wave == 0) {
-      const float gv = lane < n ? bits_to_f32(gbits, p.dtype_gb) : 0.0f;
-      const float bv = lane < n ? bits_to_f32(bbits, p.dtype_gb) : 0.0f;
-      if (v + 1 < v1) {  // next v-head's g and beta, awaited at the end of this one
-        const int64_t gi = (int64_t)(t0 + min(lane, n - 1)) * p.sgb + h + 1;
-        gnext = load_bits(p.g, gi, p.dtype_gb);
-        bnext = load_bits(p.beta, gi, p.dtype_gb);
-      }
-      float cs = gv;
-#pragma unroll
-      for (int off = 1; off < 64; off <<= 1) {
-        const float o = __shfl_up(cs, off, 64);
-        if (lane >= off) cs += o;
-      }
-      const float gl = __shfl(cs, kC - 1, 64);
-      const float gcap = __shfl(cs, cap_row, 64);
-      sGam[lane] = cs;
-      sBeta[lane] = bv;
-      sW[lane] = decay_exp(gl - cs);
-      if (chunk == cap_chunk) sWc[lane] = lane <= cap_row ? decay_exp(gcap - cs) : 0.0f;
-      const float eg = decay_exp(cs);
-      float* sc = p.sc + cv * 256;
-      sc[lane] = sInv[0][lane] * eg;
-      sc[64 + lane] = sInv[1][lane] * eg;
-      sc[128 + lane] = cs;
-      sc[192 + lane] = eg;
-    }
-    lds_barrier();
-    // 3b. A (f32) and M (CT) from the Gram tiles
-#pragma unroll
-    for (int s = 0; s < JPW; ++s) {
-      const int job = wave + kPW * s;
-      if (job >= 20) break;
-      const bool isqk = job >= 10;
-      const int idx = isqk ? job - 10 : job;
-      const int tr = idx >= 6 ? 3 : idx >= 3 ? 2 : idx >= 1 ? 1 : 0;
-      const int tc = idx - tr * (tr + 1) / 2;
-      const int c = 16 * tc + col;
-      const float gc = sGam[c];
-      // the four rows' gam and beta as vectors; the ratio is exponentiated for
-      // every element and masked afterwards (above the diagonal it may be
-      // inf, and the select keeps it out), so the block has no branches
-      const float4_t gr = *reinterpret_cast<const float4_t*>(sGam + 16 * tr + 4 * grp);
-      const float4_t br = *reinterpret_cast<const float4_t*>(sBeta + 16 * tr + 4 * grp);
+    const int buf = (v - v0) & 1;
+    const float *sGam = sGam2[buf], *sBeta = sBeta2[buf], *sW = sW2[buf], *sWc = sWc2[buf];
+    // 3b. A (f32) and M (CT) from the Gram tiles: the ratio is exponentiated
+    //     for every element and masked afterwards (above the diagonal it may
+    //     be inf, and the select keeps it out), so there are no branches
+    auto put_a = [&](int tr, int tc, const float4_t& g, const float4_t& br, const float4_t& e) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int r = 16 * tr + 4 * grp + i;
-        const float e = decay_exp(gr[i] - gc);
-        const float d = c <= r ? e : 0.0f;
-        if (!isqk)
-          sA[r * LDF + c] = c < r ? (br[i] * gram[s][i]) * d : 0.0f;
+        const int r = 16 * tr + 4 * grp + i, c = 16 * tc + col;
+        sA[r * LDF + c] = c < r ? (br[i] * g[i]) * e[i] : 0.0f;
+      }
+    };
+    auto put_m = [&](int tr, int tc, const float4_t& g, const float4_t& e) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = 16 * tr + 4 * grp + i, c = 16 * tc + col;
+        sM[r * LDT + c] = static_cast<CT>(c <= r ? g[i] * e[i] : 0.0f);
+      }
+    };
+    auto ratios = [&](const float4_t& gr, float gc) {
+      float4_t e;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) e[i] = decay_exp(gr[i] - gc);
+      return e;
+    };
+    {
+      const int tr = tile_row(wave), tc = wave - tr * (tr + 1) / 2;
+      const int xr = 3, xc = xidx - 6;
+      const float4_t gr = *reinterpret_cast<const float4_t*>(sGam + 16 * tr + 4 * grp);
+      const float4_t br = *reinterpret_cast<const float4_t*>(sBeta + 16 * tr + 4 * grp);
+      const float gc = sGam[16 * tc + col];
+      const float4_t e = ratios(gr, gc);
+      put_a(tr, tc, gkk, br, e);
+      put_m(tr, tc, gqk, e);
+      if (extra) {
+        const float4_t xg = *reinterpret_cast<const float4_t*>(sGam + 16 * xr + 4 * grp);
+        const float4_t xe = ratios(xg, sGam[16 * xc + col]);
+        if (xkk)
+          put_a(xr, xc, gx, *reinterpret_cast<const float4_t*>(sBeta + 16 * xr + 4 * grp), xe);
         else
-          sM[r * LDT + c] = static_cast<CT>(c <= r ? gram[s][i] * d : 0.0f);
+          put_m(xr, xc, gx, xe);
       }
     }
     lds_barrier();
@@ -421,13 +469,27 @@ __global__ __launch_bounds__(64 * kPW, (sizeof(CT) == 4 && DK > 64) ? 2 : 4) voi
     //     column j), rows by forward substitution.
     if (wave == 0) {
       const int b = lane >> 4, j = lane & 15;
+      // Rows are requested several ahead of their sums (as written, one or two
+      // reads were in flight and each was waited for, 1900 cycles).
       float t[16];
+      float4_t a[16][4];
+      auto load_row = [&](int r) {
+        const float* arow = sA + (16 * b + r) * LDF + 16 * b;
+#pragma unroll
+        for (int c4 = 0; c4 < 4; ++c4)
+          if (4 * c4 < r) a[r][c4] = *reinterpret_cast<const float4_t*>(arow + 4 * c4);
+      };
+#pragma unroll
+      for (int r = 1; r < 7; ++r) load_row(r);
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const float* arow = sA + (16 * b + r) * LDF + 16 * b;
+        // (at most 15 vectors in flight, for the registers)
+        constexpr int ask[16] = {0, 7, 8, 0, 9, 10, 0, 11, 12, 0, 13, 14, 15, 0, 0, 0};
+        if (ask[r]) load_row(ask[r]);
+        __builtin_amdgcn_sched_barrier(0);
         float s = (r == j) ? 1.0f : 0.0f;
 #pragma unroll
-        for (int c = 0; c < r; ++c) s = fmaf(-arow[c], t[c], s);
+        for (int c = 0; c < r; ++c) s = fmaf(-a[r][c >> 2][c & 3], t[c], s);
         t[r] = s;
       }
       float* dst = sTT + (16 * b + j) * LDF + 16 * b;
@@ -435,28 +497,43 @@ __global__ __launch_bounds__(64 * kPW, (sizeof(CT) == 4 && DK > 64) ? 2 : 4) voi
       for (int r4 = 0; r4 < 16; r4 += 4)
         *reinterpret_cast<float4_t*>(dst + r4) = float4_t{t[r4], t[r4 + 1], t[r4 + 2], t[r4 + 3]};
     }
+    if (wave == kPW - 1 && v + 1 < v1) head_rows(v + 1);
     lds_barrier();
-    //     Off-diagonal blocks, block row by block row:
-    //     T_ij = -T_ii sum_{k=j}^{i-1} A_ik T_kj   (wave j computes T_ij)
+    //     Off-diagonal blocks: T_ij = -T_ii sum_{k=j}^{i-1} A_ik T_kj.  Wave j
+    //     forms column j downwards: a finished T_kj is the next products'
+    //     operand as it stands (accumulator and B layouts agree), so nothing
+    //     passes through LDS or a barrier on the way (with both, block row by
+    //     block row, 2600 cycles).
+    if (wave < 3) {
+      const int j = wave;
+      auto a_block = [&](int i, int k) {
+        return *reinterpret_cast<const float4_t*>(sA + (16 * i + col) * LDF + 16 * k + 4 * grp);
+      };
+      float4_t a[4][3], td[4], tc[4];
 #pragma unroll
-    for (int i = 1; i < 4; ++i) {
-      if (wave < i) {
-        const int j = wave;
-        float4_t R = {0.f, 0.f, 0.f, 0.f};
-        for (int k = j; k < i; ++k) {
-          const float4_t a = *reinterpret_cast<const float4_t*>(sA + (16 * i + col) * LDF + 16 * k + 4 * grp);
-          const float4_t bt = *reinterpret_cast<const float4_t*>(sTT + (16 * j + col) * LDF + 16 * k + 4 * grp);
-          Mma<float>::mma(R, a, bt);
-        }
-        float4_t ti;
+      for (int i = 1; i < 4; ++i) {
 #pragma unroll
-        for (int s = 0; s < 4; ++s) ti[s] = sTT[(16 * i + 4 * grp + s) * LDF + 16 * i + col];
-        float4_t tij = {0.f, 0.f, 0.f, 0.f};
-        Mma<float>::mma(tij, ti, R);  // R's accumulator layout is the B operand layout
-        *reinterpret_cast<float4_t*>(sTT + (16 * j + col) * LDF + 16 * i + 4 * grp) = -tij;
+        for (int k = 0; k < i; ++k) a[i][k] = a_block(i, k);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) td[i][s] = sTT[(16 * i + 4 * grp + s) * LDF + 16 * i + col];
       }
-      lds_barrier();
+      const float4_t tjj = *reinterpret_cast<const float4_t*>(sTT + (16 * j + col) * LDF + 16 * j + 4 * grp);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) tc[k] = tjj;
+#pragma unroll
+      for (int i = 1; i < 4; ++i)
+        if (i > j) {
+          float4_t R = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int k = 0; k < i; ++k)
+            if (k >= j) Mma<float>::mma(R, a[i][k], tc[k]);
+          float4_t tij = {0.f, 0.f, 0.f, 0.f};
+          Mma<float>::mma(tij, td[i], R);
+          tc[i] = -tij;
+          *reinterpret_cast<float4_t*>(sTT + (16 * j + col) * LDF + 16 * i + 4 * grp) = tc[i];
+        }
     }
+    lds_barrier();
     // 3d. U blocks (s, b): U[slot(s, m)][token block b], as U^T = (W Tm B)^T K^
     //     on MFMA; token tiles of block b are TPK*b + u.  Tm[r][c] = 0 for
     //     r < c, so token blocks kr < b contribute nothing.
@@ -523,9 +600,7 @@ __global__ __launch_bounds__(64 * kPW, (sizeof(CT) == 4 && DK > 64) ? 2 : 4) voi
         dst[(t * NKT + b) * 64 + lane] = pack_frag(acc, 0, CT(0));
       }
     }
-    gbits = gnext;  // the loads were issued a whole v-head ago
-    bbits = bnext;
-    lds_barrier();  // before the next v-head rewrites sA, sTT, sM, sGam
+    lds_barrier();  // before the next v-head rewrites sA, sTT, sM
   }
 
 }
@@ -1334,7 +1409,8 @@ int launch_dk(const ScanParams& p, hipStream_t stream) {
   // other; where a work-group per v-head still fits the CUs once, each takes
   // one (the Gram tiles are formed again).  16 / 32 heads x 128, us: T = 100
   // f16 14.2 -> 10.8, f32 20.5 -> 15.3; T = 400 16.0 -> 12.6, 23.5 -> 18.4; at
-  // T = 600 (320 work-groups) 16.5 -> 16.0, f32 24.0 -> 30.2.
+  // T = 600 (320 work-groups) 16.5 -> 16.0, f32 24.0 -> 30.2 (the head's steps
+  // have since become shorter: T = 400 now 11.0 and 17.7, 600 15.8 and 22.8).
   const int vsplit = (int64_t)p.nchunks * p.Hv <= 256 ? p.Hv / p.Hk : 1;
   hipLaunchKernelGGL((scan_prepare<CT, IT, DK>), dim3(p.nchunks, p.Hk, vsplit), dim3(64 * kPW), 0, stream, p);
   int rc = check_launch("scan_prepare");

@@ -290,3 +290,21 @@ def test_scan_varlen_walked_in_a_row_equals_single_scans(clef, precision, dtype,
         o, _, f = scan.prefill(*(t[a:b] for t in x), initial=s0)
         assert torch.equal(out[a:b], o)
         assert torch.equal(final[s], f)
+
+
+@gpu
+@pytest.mark.parametrize("precision", ["strict", "mixed"])
+@pytest.mark.parametrize("Hv", [1, 3, 5])
+def test_scan_heads_of_one_key_head_in_turn(clef, precision, Hv):
+    """A k-head's v-heads prepared one after the other (each one's decay formed
+    during the one before): every head equals the same head scanned alone."""
+    T, dk, dv = 5440 if Hv == 3 else 3400, 32, 16
+    dt = torch.float32 if precision == "strict" else torch.float16
+    q, k, v, g, beta = case_inputs(16, T, 1, Hv, dk, dv, dtype=dt)
+    scan = clef.DeltaScan(dk, dv, precision)
+    out, cap, fin = scan.prefill(q, k, v, g, beta, capture=130)
+    for h in range(Hv):
+        o, c, f = scan.prefill(q, k, v[:, h:h + 1].contiguous(), g[:, h:h + 1].contiguous(),
+                               beta[:, h:h + 1].contiguous(), capture=130)
+        assert torch.equal(out[:, h:h + 1], o)
+        assert torch.equal(cap[h:h + 1], c) and torch.equal(fin[h:h + 1], f)
