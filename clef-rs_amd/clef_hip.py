@@ -267,7 +267,7 @@ def _rows(t, name):
 def gemm(x, w, out=None, out_dtype=None, residual=None):
     """y = x . w^T (GemmKernel::forward, neural.rs:50-55).
 
-    x [M,K], w [N,K] share a dtype (f16: f16 MFMA; f32: f32 MFMA), f32
+    x [M,K], w [N,K] share a dtype (f16, or f32 by exact bf16 splits), f32
     accumulation.  With `residual` (an f32 [M,N] tensor) the rounded product
     is added into it in place and `residual` is returned.
     """

@@ -253,7 +253,8 @@ constexpr int kPW = 8;  // waves of a scan_prepare work-group
 // waves idle; at T = 4096 two work-groups of two heads run twice on each CU.
 // The next head's decay beside this one's inversion, a tile position's A and M
 // on one wave, reads of the inversion requested ahead and its off-diagonal
-// blocks without barriers took 12100 of 31800 cycles to 7500 of 27000 (f16).
+// blocks without barriers shortened it: the first three took a work-group's
+// 31800 cycles (f16, two heads; these steps 17400) to 27500 (12200).
 // 16 / 32 heads x 128, us, f16 and f32: T = 4096 37.5 -> 33.8, 88.7 -> 82.3;
 // T = 1000 18.0 -> 16.2, 24.6 -> 22.8; T = 100 10.8 -> 8.8, 15.3 -> 14.4.
 //

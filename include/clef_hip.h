@@ -141,7 +141,7 @@ int clef_delta_scan_varlen(const void* q, const void* k, const void* v, int64_t 
  * Replaces GemmKernel::forward / "clef-metal4-gemm" (neural.rs:50-55,
  * 151-173; neural.metal:72-97) and candle_nn::Linear (projection.rs:82-95).
  * dtype_in CLEF_F16: f16 operands on f16 MFMA, f32 accumulation;
- * CLEF_F32: f32 operands on f32 MFMA.  x and W share dtype_in.
+ * CLEF_F32: f32 products and sums.  x and W share dtype_in.
  * epilogue: CLEF_EPI_STORE writes y in dtype_out (f16 output is rounded once
  * from the f32 accumulator, as neural.metal:23-26);
  * CLEF_EPI_RESIDUAL adds the (dtype_out-rounded) product into an f32 residual
@@ -279,7 +279,7 @@ int clef_values_transposed(const void* x, int64_t ldx, int dtype_in, void* y, in
  * q [heads, ldq_tok, d] (rows 0..qn-1), k [kv_heads, ldk_tok, d],
  * vt [kv_heads, d, ldv_tok] (from clef_values_transposed); gate token stride
  * ldg and head stride hsg; y [qn, heads*d] token stride ldy.  dtype is the
- * operand dtype of q/k/v/gate (f16: f16 MFMA, f32: f32 MFMA), accumulation
+ * operand dtype of q/k/v/gate (f16 products, f32 products), accumulation
  * and softmax in f32; y in dtype (the product of the rounded attention and
  * the rounded gate, as the reference's mixed profile does).  d in {64, 128,
  * 256}; heads % kv_heads == 0; qn <= kn.
@@ -349,7 +349,7 @@ int clef_head_logits(const float* x, int H, const float* w, int n_logits, float*
  * attention layer FullAttention::forward (:451-525).  Layer kinds: 0 =
  * linear_attention (DeltaNet), 1 = full_attention.
  *
- * Profiles: CLEF_PROFILE_F32 runs every projection on f32 MFMA and the strict
+ * Profiles: CLEF_PROFILE_F32 runs every projection in f32 and the strict
  * scan (the reference's CPU/Metal F32 profile); CLEF_PROFILE_MIXED_F16 runs
  * f16 projections with f32 accumulation and the reference's half rounding
  * points, an f32 residual stream, and the scan in `scan_precision`.
