@@ -139,20 +139,31 @@ __device__ __forceinline__ float bits_to_f32(uint32_t b, int dtype) {
 // full precision; results below the normal range may flush to zero.
 __device__ __forceinline__ float decay_exp(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504088896341f); }
 
-// Inclusive running sum over the 64 lanes by DPP moves: within rows of 16
-// (shifts by 1, 2, 4, 8, zeros in), then each row's total into the rows after it.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ float dpp_or_zero(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xf, false));
+// Inclusive running sum over the 64 lanes: each step adds the partial sum 1, 2,
+// 4, ... 32 lanes below, so a lane's partials are sums of its 2, 4, ... last
+// values.  (Summing the rows of 16 first and adding their totals is shorter but
+// rounds differently, which moves every result of the half-precision profile.)
+// By DPP moves and row swaps: a shuffle through LDS per step takes longer than
+// the 16 x 16 inversion this runs beside.
+__device__ __forceinline__ uint32_t lane_below(uint32_t v) {  // of lane l - 1, 0 into lane 0
+  return __builtin_amdgcn_update_dpp(0, v, 0x138, 0xf, 0xf, false);  // wave_shr:1
 }
-__device__ __forceinline__ float wave_running_sum(float v) {
-  v += dpp_or_zero<0x111, 0xf>(v);  // row_shr:1
-  v += dpp_or_zero<0x112, 0xf>(v);  // row_shr:2
-  v += dpp_or_zero<0x114, 0xf>(v);  // row_shr:4
-  v += dpp_or_zero<0x118, 0xf>(v);  // row_shr:8
-  v += dpp_or_zero<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
-  v += dpp_or_zero<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
-  return v;
+__device__ __forceinline__ float wave_running_sum(float v, int lane) {
+#pragma unroll
+  for (int off = 1; off < 16; off <<= 1) {
+    uint32_t b = __float_as_uint(v);
+#pragma unroll
+    for (int i = 0; i < off; ++i) b = lane_below(b);
+    v += __uint_as_float(b);
+  }
+  // of lane l - 16: rows 0 and 2 into rows 1 and 3, row 1 into row 2
+  const uint32_t b = __float_as_uint(v);
+  const auto r = __builtin_amdgcn_permlane16_swap(b, b, false, false);           // rows 0 0 2 2 and 1 1 3 3
+  const auto r1 = __builtin_amdgcn_permlane32_swap(r[1], r[1], false, false)[0];  // rows 1 1 1 1
+  v += lane < 16 ? 0.0f : __uint_as_float((lane >> 4) == 2 ? r1 : r[0]);
+  const uint32_t c = __float_as_uint(v);
+  const uint32_t lo = __builtin_amdgcn_permlane32_swap(c, c, false, false)[0];  // rows 0 1 0 1
+  return v + (lane < 32 ? 0.0f : __uint_as_float(lo));
 }
 
 __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
@@ -373,8 +384,7 @@ __global__ __launch_bounds__(64 * kPW, (sizeof(CT) == 4 && DK > 64) ? 2 : 4) voi
   // token): the carry's row factors 1/|k| e^gam (for V - e^gam K^ S) and
   // qscale/|q| e^gam (for e^gam Q^ S), gam (capture) and e^gam.  The first
   // v-head's here, the next one's while wave 0 inverts a head's diagonal
-  // blocks; the running sum moves by DPP (six shuffles through LDS took as
-  // long as that inversion).
+  // blocks.
   auto head_rows = [&](int v) {
     const int h = hk * rep + v, buf = (v - v0) & 1;
     const float gv = lane < n ? bits_to_f32(gbits, p.dtype_gb) : 0.0f;
@@ -384,7 +394,7 @@ __global__ __launch_bounds__(64 * kPW, (sizeof(CT) == 4 && DK > 64) ? 2 : 4) voi
       gbits = load_bits(p.g, gi, p.dtype_gb);
       bbits = load_bits(p.beta, gi, p.dtype_gb);
     }
-    const float cs = wave_running_sum(gv);
+    const float cs = wave_running_sum(gv, lane);
     const float gl = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cs), kC - 1));
     sGam2[buf][lane] = cs;
     sBeta2[buf][lane] = bv;

@@ -308,3 +308,37 @@ def test_scan_heads_of_one_key_head_in_turn(clef, precision, Hv):
                                beta[:, h:h + 1].contiguous(), capture=130)
         assert torch.equal(out[:, h:h + 1], o)
         assert torch.equal(cap[h:h + 1], c) and torch.equal(fin[h:h + 1], f)
+
+
+@gpu
+def test_scan_decay_is_summed_by_doubling_windows(clef):
+    """The cumulative log-decay of a chunk adds partial sums 1, 2, ... 32 tokens back, in f32.
+    With no keys the output is e^gam of the initial state; large opposite decays beside the
+    16-token marks make any other order visible (up to 4e-6 of e^gam; the exponential and the
+    output's roundings are 4 of 2^-24 times |gam| + 1)."""
+    T, H, d, chunks = 64, 8, 32, 3
+    rng = np.random.default_rng(17)
+    g = -rng.uniform(0.0, 0.1, (chunks * T, H)).astype(np.float32)
+    for c in range(chunks):
+        for t, size in ((15, 75), (31, 70), (47, 65), (7, 30), (22, 40)):
+            s = rng.uniform(0.9, 1.1, H) * size
+            g[c * T + t] = -s
+            g[c * T + t + 1] = s
+    gam = g.reshape(chunks, T, H).copy()
+    for off in (1, 2, 4, 8, 16, 32):
+        gam[:, off:] = gam[:, off:] + gam[:, :-off]
+    gam = gam.astype(np.float64)
+    gam[1:] += np.cumsum(gam[:-1, -1:], axis=0)  # the carry multiplies the chunks' decays
+    q = torch.zeros((chunks * T, H, d), device="cuda")
+    q[:, :, 0] = 1.0
+    zero = torch.zeros((chunks * T, H), device="cuda")
+    init = torch.ones((H, d, d), device="cuda")
+    scan = clef.DeltaScan(d, d, "strict")
+    args = (q, torch.zeros_like(q), torch.zeros_like(q))
+    base = scan.prefill(*args, zero, zero, initial=init)[0].double().cpu().numpy()
+    out = scan.prefill(*args, torch.from_numpy(g).cuda(), zero, initial=init)[0].double().cpu().numpy()
+    exp = np.exp(gam).reshape(chunks * T, H)[..., None]
+    rel = np.abs(out / base / exp - 1.0)
+    tol = 2.0 ** -22 * (np.abs(gam).reshape(chunks * T, H)[..., None] + 4.0)
+    small = np.abs(gam).reshape(chunks * T, H) < 5.0
+    assert (rel <= tol)[small].all(), rel[small].max()
