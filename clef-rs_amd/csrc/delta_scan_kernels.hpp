@@ -32,6 +32,7 @@
 #include "common.hpp"
 #include "ragged.hpp"
 #include "scan.hpp"
+#include "scan_walk.hpp"
 
 namespace clef {
 
@@ -1291,10 +1292,11 @@ __device__ __forceinline__ void carry_outputs(const ScanParams& p, const CarryCt
 // batch, a work-group per sequence; 3: a ragged batch, a work-group walks all
 // sequences' chunks in token order.
 // Bound: the recurrence's serial chain, about 1 us a chunk (f16, dk 128).  One
-// work-group fills a CU's LDS, so with 256 or more (head, columns) the batch's
-// sequences take turns on a CU, and in MODE 2 each turn starts with an empty
+// work-group fills a CU (its LDS or its registers), so with 256 or more (head,
+// columns) the batch's sequences take turns on a CU, and in MODE 2 each turn starts with an empty
 // ring and register pipeline, about 5 us.  MODE 3 keeps both full across the
-// boundaries (a boundary costs 0.7 us, the states out and in).  32 heads x 128,
+// boundaries (a boundary costs 0.7 us, the states out and in), but it takes
+// whole rounds of the batch (which of the two: scan_walk.hpp).  32 heads x 128,
 // us: 8 sequences of 64-1200 tokens, 5003 in all, f16 119 -> 85, f32 423 -> 380;
 // 16 of 12 tokens 90 -> 24, 168 -> 89; 64 of 64 tokens 372 -> 114, 743 -> 340;
 // 1200 + 800 tokens 43 -> 36, 160 -> 156; 32 of 128-4096 tokens, 58786 in all,
@@ -1422,16 +1424,14 @@ int launch_dk(const ScanParams& p, hipStream_t stream) {
   // f16 14.2 -> 10.8, f32 20.5 -> 15.3; T = 400 16.0 -> 12.6, 23.5 -> 18.4; at
   // T = 600 (320 work-groups) 16.5 -> 16.0, f32 24.0 -> 30.2 (the head's steps
   // have since become shorter: T = 400 now 11.0 and 17.7, 600 15.8 and 22.8).
-  const int vsplit = (int64_t)p.nchunks * p.Hv <= 256 ? p.Hv / p.Hk : 1;
+  const int vsplit = (int64_t)p.nchunks * p.Hv <= device_cus() ? p.Hv / p.Hk : 1;
   hipLaunchKernelGGL((scan_prepare<CT, IT, DK>), dim3(p.nchunks, p.Hk, vsplit), dim3(64 * kPW), 0, stream, p);
   int rc = check_launch("scan_prepare");
   if (rc) return rc;
   const int ntiles = (p.dv + kVT - 1) / kVT;
   const int nseq = p.seq_tab ? p.nseq : 1;
   const dim3 block(Carry<CT, IT, DK>::THREADS);
-  // a batch walks in a row where its (head, columns) fill the CUs; with fewer,
-  // sequences side by side use the idle ones
-  if (p.seq_tab && p.Hv * ntiles >= device_cus())
+  if (p.seq_tab && scan_walks_in_a_row(p.Hv * ntiles, device_cus(), p.T, nseq, sizeof(CT) == 2))
     hipLaunchKernelGGL((scan_carry<CT, IT, DK, 3>), dim3(p.Hv * ntiles), block, 0, stream, p);
   else if (p.seq_tab)
     hipLaunchKernelGGL((scan_carry<CT, IT, DK, 2>), dim3(nseq * p.Hv * ntiles), block, 0, stream, p);

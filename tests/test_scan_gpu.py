@@ -10,6 +10,8 @@ JSON file named by CLEF_PARITY_LOG.
 """
 import json
 import os
+import pathlib
+import subprocess
 
 import numpy as np
 import pytest
@@ -290,6 +292,53 @@ def test_scan_varlen_walked_in_a_row_equals_single_scans(clef, precision, dtype,
         o, _, f = scan.prefill(*(t[a:b] for t in x), initial=s0)
         assert torch.equal(out[a:b], o)
         assert torch.equal(final[s], f)
+
+
+def _check_varlen_equals_single(clef, precision, dtype, Hk, Hv, dk, dv, lens):
+    x = case_inputs(18, sum(lens), Hk, Hv, dk, dv, dtype=dtype)
+    cu = torch.tensor(np.concatenate([[0], np.cumsum(lens)]), dtype=torch.int32, device="cuda")
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    init = 0.1 * torch.randn((len(lens), Hv, dk, dv), generator=gen, device="cuda")
+    scan = clef.DeltaScan(dk, dv, precision)
+    out, final = scan.prefill_varlen(*x, cu, initial=init)
+    for s, (a, b) in enumerate(zip(cu[:-1].tolist(), cu[1:].tolist())):
+        o, _, f = scan.prefill(*(t[a:b] for t in x), initial=init[s])
+        assert torch.equal(out[a:b], o)
+        assert torch.equal(final[s], f)
+
+
+@gpu
+@pytest.mark.parametrize("precision,dtype", [("mixed", torch.float16), ("strict", torch.float32)])
+@pytest.mark.parametrize("Hk,Hv,dk,dv", [(16, 48, 128, 128), (17, 34, 64, 120)])
+@pytest.mark.parametrize("lens", [[12, 64, 100, 1], [1500, 70, 900]])
+def test_scan_varlen_more_groups_than_cus(clef, precision, dtype, Hk, Hv, dk, dv, lens):
+    """Two rounds of work-groups, the second partly empty, and a last column tile that is
+    not whole: short sequences walk in a row, long ones side by side; each equals the
+    sequence scanned alone."""
+    _check_varlen_equals_single(clef, precision, dtype, Hk, Hv, dk, dv, lens)
+
+
+def test_scan_walk_rule(tmp_path):
+    """The rule alone, on the host: whole rounds walk in a row, part rounds only short
+    sequences, fewer groups than CUs never."""
+    src, exe = tmp_path / "rule.cpp", tmp_path / "rule"
+    src.write_text('#include <cstdio>\n#include <cstdlib>\n#include "scan_walk.hpp"\n'
+                   "int main(int, char** a) { std::printf(\"%d\", clef::scan_walks_in_a_row(std::atoi(a[1]), 256, "
+                   "std::atoi(a[2]) * std::atoi(a[3]), std::atoi(a[3]), std::atoi(a[4]) != 0)); }\n")
+    csrc = pathlib.Path(__file__).resolve().parents[1] / "clef-rs_amd" / "csrc"
+    subprocess.run(["g++", "-std=c++17", f"-I{csrc}", str(src), "-o", str(exe)], check=True)
+
+    def walks(groups, tokens, nseq, f16):
+        return subprocess.run([str(exe)] + [str(int(v)) for v in (groups, tokens, nseq, f16)],
+                              check=True, capture_output=True, text=True).stdout == "1"
+
+    for f16 in (False, True):
+        for tokens, nseq in ((1, 1), (64, 64), (2550, 32), (32768, 1)):
+            assert walks(256, tokens, nseq, f16) and walks(512, tokens, nseq, f16)
+            assert not walks(255, tokens, nseq, f16)
+        assert walks(384, 12, 16, f16)
+        for groups in (264, 288, 384):
+            assert not walks(groups, 4096, 8, f16) and not walks(groups, 2550, 32, f16)
 
 
 @gpu
