@@ -12,8 +12,12 @@
 // K = 64 0.58e-7 (f32 MFMA kernel 1.31e-7), K = 320 0.67e-7 (1.20e-7), K =
 // 2048 1.07e-7 (1.79e-7), K = 6144 1.68e-7 (2.74e-7); without the groups 1.60
 // and 2.69e-7 at the last two.
-// Tiles with values that the split does not hold (tiny, infinite, NaN) are
-// formed on the f32 MFMA instead, at the end.
+// Outputs that the split does not hold (not finite, or where values below
+// 2^-100 matter) are formed on the f32 MFMA instead, at the end, their 16 x 16
+// blocks dealt to all waves.  At 2048 x 8192 x 2048 (f32 MFMA kernel 654 us,
+// here 367): one such weight 382, one such value in every x row 426, one
+// infinity 490, a whole x row of such values 556; where every output is one,
+// 2.1 ms.
 //
 // The tile's x and weight rows pass through registers (loaded D stages
 // ahead), where they are split, into two LDS buffers of three planes each.
@@ -40,29 +44,30 @@ namespace {
 
 typedef uint32_t uint4_t __attribute__((ext_vector_type(4)));
 
-// Stores four consecutive columns c .. c + 3 of row r, clipped to M x N.
-__device__ __forceinline__ void store_row4(const GemmParams& p, int r, int c, const float4_t& o, bool yvec) {
-  if (r >= p.M) return;
+// Stores four consecutive columns c .. c + 3 of row r: as a vector (`whole`), or
+// one by one those within N and not in the mask `skip`.
+__device__ __forceinline__ void store_row4(const GemmParams& p, int r, int c, const float4_t& o, bool whole,
+                                           uint32_t skip) {
   const int64_t off = (int64_t)r * p.ldy + c;
   if (p.dtype_out == 1) {
     const half4 h = {static_cast<half_t>(o[0]), static_cast<half_t>(o[1]), static_cast<half_t>(o[2]),
                      static_cast<half_t>(o[3])};
     half_t* dst = static_cast<half_t*>(p.y) + off;
-    if (yvec && c + 3 < p.N) {
+    if (whole) {
       *reinterpret_cast<half4*>(dst) = h;
     } else {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        if (c + e < p.N) dst[e] = h[e];
+        if (c + e < p.N && !(skip >> e & 1)) dst[e] = h[e];
     }
   } else {
     float* dst = static_cast<float*>(p.y) + off;
-    if (yvec && c + 3 < p.N) {
+    if (whole) {
       *reinterpret_cast<float4_t*>(dst) = o;
     } else {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        if (c + e < p.N) dst[e] = o[e];
+        if (c + e < p.N && !(skip >> e & 1)) dst[e] = o[e];
     }
   }
 }
@@ -82,7 +87,10 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_split(GemmParams p) {
   static_assert(!FAST || (U == 1 && D == 1), "the interleaved loop is one sub-stage deep");
   static_assert(2 * kBuf * 2 + 16 <= 160 * 1024, "LDS");
   __shared__ __attribute__((aligned(16))) __bf16 smem[2 * kBuf];
-  __shared__ int tiny_flag;
+  // of [x rows | weight rows], formed only if the tile met a value below 2^-100:
+  // K 2^-97 if the row holds one, else 0; its largest magnitude
+  __shared__ float row_tiny[ROWS], row_max[ROWS];
+  __shared__ int any_tiny, any_redo;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -150,6 +158,7 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_split(GemmParams p) {
   // 16-byte chunk c of row r at c ^ ((r >> 2) & 3) (16 consecutive rows of
   // one chunk, and 4 rows of all four, cover the 64 banks once)
   uint32_t smallest = 0xffffffffu;  // of |x| > 0, as 2 * bits - 1
+  constexpr uint32_t kTiny = (27u << 24) - 1u;  // of 2^-100
   auto split = [&](int st, int d) {
     const bool whole = (st + 1) * U * 32 <= p.K;
     __bf16* const buf = smem + (st & 1) * kBuf;
@@ -235,7 +244,7 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_split(GemmParams p) {
     }
   };
 
-  if (tid == 0) tiny_flag = 0;
+  if (tid == 0) any_tiny = any_redo = 0;
   load(0, 0);
   if (D == 2 && nst > 1) load(1, 1);
   split(0, 0);
@@ -328,27 +337,59 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_split(GemmParams p) {
   }
   if (active) fold();
 
-  // Values the split does not hold: below 2^-100 the low parts leave bf16's
-  // range; infinities, NaN and values that round to infinity make every
-  // output they meet NaN.  Such tiles are formed again on f32 products.
-  if (smallest < (27u << 24) - 1u) tiny_flag = 1;
+  // Values the split does not hold.  Below 2^-100 the low parts leave bf16's
+  // range: the term errs by up to 2^-124 of the other factor.  Infinities, NaN
+  // and values that round to infinity make every output they meet NaN.  An
+  // output that is not finite, or smaller than K 2^-97 of the largest factor
+  // that such a small value of its x row or weight row may meet (larger ones
+  // err by less than 2^-27), is formed again on f32 products.  That follows
+  // from the row, the column and the result alone, so a row's bits do not
+  // depend on what shares its tile.
+  if (smallest < kTiny) any_tiny = 1;
   lds_barrier();
-  if (!active) return;
-  bool again = tiny_flag != 0;
+  const bool tiny = __builtin_amdgcn_readfirstlane(any_tiny) != 0;
+  if (tiny) {
+    // the rows once more, four of them a wave at a time
+    const int rl = lane >> 4, cl = 4 * (lane & 15);
+    for (int row = 4 * wave + rl; row < ROWS; row += 32) {
+      const bool is_x = row < BM;
+      const int rb = row - BM;
+      const float* op = is_x ? X : EPI == 2 && (rb & 16) ? W2 : W;
+      const int r = is_x ? min(m0 + row, p.M - 1) : min(n0 + (EPI == 2 ? (rb >> 5) * 16 + (rb & 15) : rb), p.N - 1);
+      const float* src = op + (int64_t)r * (is_x ? p.ldx : p.ldw);
+      float m = 0.0f;
+      uint32_t least = 0xffffffffu;
+      for (int k0 = 0; k0 < p.K; k0 += 512) {
+        float4_t v[8];
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
+        for (int u = 0; u < 8; ++u) v[u] = *reinterpret_cast<const float4_t*>(src + min(k0 + 64 * u + cl, p.K - 4));
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
+        for (int u = 0; u < 8; ++u)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) again |= !(fabsf(tot[i][j][e]) < __builtin_inff());
-  again = __ballot(again) != 0;
+          for (int e = 0; e < 4; ++e) {
+            m = fmaxf(m, fabsf(v[u][e]));
+            least = min(least, 2u * __float_as_uint(v[u][e]) - 1u);
+          }
+      }
+      m = lane_max<16>(m);
+      const float t = lane_max<16>(least < kTiny ? static_cast<float>(p.K) * 0x1p-97f : 0.0f);
+      if (cl == 0) row_max[row] = m, row_tiny[row] = t;
+    }
+    lds_barrier();
+  }
 
   const int esz = (EPI == 1 || p.dtype_out != 1) ? 4 : 2;
   const bool yvec = ((reinterpret_cast<uintptr_t>(p.y) | (uintptr_t)(p.ldy * esz)) & (4 * esz - 1)) == 0;
-  const int orow = m0 + wm * WM + r16, ocol = n0 + wn * (EPI == 2 ? WN / 2 : WN) + 4 * c16;
   constexpr int TO = EPI == 2 ? TN / 2 : TN;
-  auto finish = [&](int i, int j, float4_t v, const float4_t& up) {
-    const int r = orow + 16 * i, c = ocol + 16 * j;
+  constexpr int NBLK = TM * TO;  // 16 x 16 output blocks of a wave
+  static_assert(NBLK <= 16, "a lane's outputs fit a 64-bit mask");
+  // block (i, j) of wave w: the lane's row and its first column
+  auto orow = [&](int w, int i) { return m0 + w / VN * WM + 16 * i + r16; };
+  auto ocol = [&](int w, int j) { return n0 + w % VN * (EPI == 2 ? WN / 2 : WN) + 16 * j + 4 * c16; };
+  // the lane's four outputs from column c of row r, without those in `skip`
+  auto finish = [&](int r, int c, float4_t v, const float4_t& up, uint32_t skip) {
+    if (r >= p.M) return;
+    const bool whole = yvec && c + 3 < p.N && skip == 0;
     if constexpr (EPI == 2) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -360,12 +401,11 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_split(GemmParams p) {
           v[e] = (v[e] / (1.0f + expf(-v[e]))) * up[e];
         }
       }
-      store_row4(p, r, c, v, yvec);
-    } else if constexpr (EPI == 1) {
-      if (r >= p.M) return;
+    }
+    if constexpr (EPI == 1) {
       float* dst = static_cast<float*>(p.y) + (int64_t)r * p.ldy + c;
       auto rd = [&](float x) { return p.dtype_out == 1 ? static_cast<float>(static_cast<half_t>(x)) : x; };
-      if (yvec && c + 3 < p.N) {
+      if (whole) {
         float4_t h = *reinterpret_cast<const float4_t*>(dst);
 #pragma unroll
         for (int e = 0; e < 4; ++e) h[e] += rd(v[e]);
@@ -373,47 +413,102 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_split(GemmParams p) {
       } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          if (c + e < p.N) dst[e] += rd(v[e]);
+          if (c + e < p.N && !(skip >> e & 1)) dst[e] += rd(v[e]);
       }
     } else {
-      store_row4(p, r, c, v, yvec);
+      store_row4(p, r, c, v, whole, skip);
     }
   };
-  if (!again) {
+  bool odd_any = tiny;
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) odd_any |= !(fabsf(tot[i][j][e]) < __builtin_inff());
+  uint64_t redo = 0;  // bit 4 (i TO + j) + e
+  if (active && __ballot(odd_any) != 0) {
+    const int xr = wm * WM + r16, wr = BM + wn * WN + 4 * c16;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TO; ++j) {
+        const int j0 = EPI == 2 ? 2 * j : j, j1 = EPI == 2 ? 2 * j + 1 : j;
+        uint32_t odd = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          auto again = [&](int jj) {
+            const float a = fabsf(tot[i][jj][e]);
+            if (!tiny) return !(a < __builtin_inff());
+            const int x = xr + 16 * i, w = wr + 16 * jj + e;
+            return !(a < __builtin_inff()) || a < row_tiny[x] * row_max[w] + row_tiny[w] * row_max[x];
+          };
+          odd |= (again(j0) || (EPI == 2 && again(j1)) ? 1u : 0u) << e;
+        }
+        redo |= (uint64_t)odd << (4 * (i * TO + j));
+        finish(orow(wave, i), ocol(wave, j), tot[i][j0], tot[i][j1], odd);
+      }
+  } else if (active) {
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TO; ++j)
-        finish(i, j, tot[i][EPI == 2 ? 2 * j : j], tot[i][EPI == 2 ? 2 * j + 1 : j]);
-    return;
+        finish(orow(wave, i), ocol(wave, j), tot[i][EPI == 2 ? 2 * j : j], tot[i][EPI == 2 ? 2 * j + 1 : j], 0);
   }
+  uint64_t* const masks = reinterpret_cast<uint64_t*>(smem);  // (no longer read) by wave and lane
+  masks[tid] = redo;
+  if (__ballot(redo != 0) != 0 && lane == 0) any_redo = 1;
+  lds_barrier();
+  if (any_redo == 0) return;
+
   // one 16 x 16 block on v_mfma_f32_16x16x4_f32, operands straight from memory
+  // (64 columns of K in registers while the 64 before are multiplied)
   auto exact = [&](const float* w, int xr, int wr) __attribute__((always_inline)) {
     float4_t s = {0.f, 0.f, 0.f, 0.f};
-    const float* xp = X + (int64_t)min(xr + r16, p.M - 1) * p.ldx;
-    const float* wp = w + (int64_t)min(wr + r16, p.N - 1) * p.ldw;
-    for (int k0 = 0; k0 < p.K; k0 += 32) {
-      float4_t a = {0.f, 0.f, 0.f, 0.f};
+    const float* xp = X + (int64_t)min(xr, p.M - 1) * p.ldx + 4 * c16;
+    const float* wp = w + (int64_t)min(wr, p.N - 1) * p.ldw + 4 * c16;
+    float4_t xv[2][4], wv[2][4];
+    auto fetch = [&](int k0, float4_t* xd, float4_t* wd) {
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
-        const int k = k0 + 16 * kb + 4 * c16;
-        float4_t xv = {0.f, 0.f, 0.f, 0.f}, wv = xv;
-        if (k < p.K) {
-          xv = *reinterpret_cast<const float4_t*>(xp + k);
-          wv = *reinterpret_cast<const float4_t*>(wp + k);
-        }
-        Mma<float>::mma(a, wv, xv);
+      for (int u = 0; u < 4; ++u) {  // past K: the row's first elements, zeroed by the products
+        const int k = k0 + 16 * u + 4 * c16 < p.K ? k0 + 16 * u : -4 * c16;
+        xd[u] = *reinterpret_cast<const float4_t*>(xp + k);
+        wd[u] = *reinterpret_cast<const float4_t*>(wp + k);
       }
-      s += a;
+    };
+    auto multiply = [&](int k0, float4_t* xd, float4_t* wd) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (k0 + 32 * h >= p.K) break;
+        float4_t a = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 2 * h; u < 2 * h + 2; ++u) {
+          const bool in = k0 + 16 * u + 4 * c16 < p.K;
+          const float4_t z = {0.f, 0.f, 0.f, 0.f};
+          Mma<float>::mma(a, in ? wd[u] : z, in ? xd[u] : z);
+        }
+        s += a;
+      }
+    };
+    fetch(0, xv[0], wv[0]);
+    for (int k0 = 0; k0 < p.K; k0 += 128) {
+      fetch(k0 + 64, xv[1], wv[1]);
+      multiply(k0, xv[0], wv[0]);
+      fetch(k0 + 128, xv[0], wv[0]);
+      multiply(k0 + 64, xv[1], wv[1]);
     }
     return s;
   };
-  for (int i = 0; i < TM; ++i)
-    for (int j = 0; j < TO; ++j) {
-      const int xr = m0 + wm * WM + 16 * i, wr = ocol - 4 * c16 + 16 * j;
-      const float4_t v = exact(W, xr, wr);
-      finish(i, j, v, EPI == 2 ? exact(W2, xr, wr) : v);
-    }
+  // the blocks dealt to all eight waves
+  for (int b = wave; b < VM * VN * NBLK; b += 8) {
+    const int w = b / NBLK, blk = b % NBLK;
+    const uint32_t odd = (uint32_t)(masks[w * 64 + lane] >> (4 * blk)) & 15u;
+    if (__ballot(odd != 0) == 0) continue;
+    const int r = orow(w, blk / TO), c = ocol(w, blk % TO), wr = c - 4 * c16 + r16;
+    const float4_t v = exact(W, r, wr);
+    const float4_t up = EPI == 2 ? exact(W2, r, wr) : v;
+    if (odd) finish(r, c, v, up, odd ^ 15u);
+  }
 }
 
 }  // namespace

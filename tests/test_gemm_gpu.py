@@ -343,6 +343,59 @@ def test_gemm_f32_split_special_values(clef, M):
 
 
 @gpu
+@pytest.mark.parametrize("M,N,K", [(33, 2048, 6144), (33, 8192, 100), (200, 8192, 64), (500, 2048, 260)])
+def test_gemm_f32_rows_do_not_depend_on_their_neighbours(clef, M, N, K):
+    """A call's rows equal those of a call on larger tiles bit for bit with values below
+    2^-100, infinities and NaN in other rows and columns as well as their own, for each
+    epilogue; rows and columns without such values equal those of a call without any."""
+    x, w = _inputs(41, M, N, K, torch.float32)
+    _, u = _inputs(42, 1, N, K, torch.float32)
+    plain = clef.gemm(x, w)
+    x[3, 5], x[7, 9], x[11, 2] = 1e-33, float("inf"), 1e-40
+    w[0, 0], w[70, 1], w[200, 3] = 1e-31, float("nan"), -1e-38
+    u[1, 2] = 1e-35
+    xl = torch.cat([x, _inputs(43, 4096 - M, 1, K, torch.float32)[0]])
+    xl[M + 1, 0], xl[-1, 1] = 1e-32, float("nan")
+
+    def same(a, b):
+        return torch.equal(torch.nan_to_num(a, nan=1e30), torch.nan_to_num(b, nan=1e30))
+
+    y = clef.gemm(x, w)
+    assert same(y, clef.gemm(xl, w)[:M])
+    assert same(clef.gemm_swiglu(x, w, u), clef.gemm_swiglu(xl, w, u)[:M])
+    h0 = torch.randn((4096, N), device="cuda")
+    assert same(clef.gemm(x, w, residual=h0[:M].clone()), clef.gemm(xl, w, residual=h0.clone())[:M])
+    assert same(clef.gemm(x, w, residual=h0[:M].clone()), h0[:M] + y)
+    assert same(clef.gemm(x, w, out_dtype=torch.float16), y.half())
+    rows = torch.ones(M, dtype=torch.bool)
+    cols = torch.ones(N, dtype=torch.bool)
+    rows[[3, 7, 11]] = False
+    cols[[0, 70, 200]] = False
+    assert torch.equal(y[rows][:, cols], plain[rows][:, cols])
+    # strided outputs: the repeated elements go where they belong and nowhere else
+    buf = torch.full((M + 2, N + 15), 7.0, device="cuda")
+    clef.gemm(x, w, out=buf[:M, 5:5 + N])
+    assert same(buf[:M, 5:5 + N], y)
+    assert (buf[M:] == 7).all() and (buf[:, :5] == 7).all() and (buf[:, 5 + N:] == 7).all()
+
+
+@gpu
+@pytest.mark.parametrize("M", [33, 300, 2048])
+def test_gemm_f32_small_terms_alone_keep_their_precision(clef, M):
+    """Rows and columns whose products are all far below 2^-100: each term is one product,
+    rounded once (and the other terms of those rows and columns as usual)."""
+    N, K = 8192, 96
+    x, w = _inputs(44, M, N, K, torch.float32)
+    x[5], w[9] = 0.0, 0.0
+    x[5, 40], w[9, 7] = 1.2345678e-34, -7.654321e-33
+    y = clef.gemm(x, w).double()
+    row, col = x[5, 40].double() * w[:, 40].double(), w[9, 7].double() * x[:, 7].double()
+    row[9] = col[5] = 0.0
+    assert ((y[5] - row).abs() <= 2.0 ** -23 * row.abs() + 2.0 ** -149).all()
+    assert ((y[:, 9] - col).abs() <= 2.0 ** -23 * col.abs() + 2.0 ** -149).all()
+
+
+@gpu
 @pytest.mark.parametrize("M,N,K", [(1000, 6144, 128), (700, 6144, 64), (1024, 6100, 192), (3000, 6144, 64)])
 def test_swiglu_192_wide_tiles(clef, M, N, K):
     """256 x 192 tiles (96 outputs): whole and ragged rows and columns, one to
