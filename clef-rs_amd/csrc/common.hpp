@@ -158,6 +158,7 @@ __device__ __forceinline__ float delta_strength(float b) { return 1.0f / (1.0f +
 void set_error(const std::string& msg);
 int fail(int code, const std::string& msg);  // records msg, returns code
 int check_launch(const char* what);          // hipGetLastError -> 0 or >0
+int device_cus();                            // CUs of the current device (cached per device; gemm_f16.hip)
 
 // Token embedding fused with the first layer's input RMSNorm (pointwise.hip):
 // writes the f32 residual rows h [T, H] and the normalised rows y (ldy apart).

@@ -35,8 +35,6 @@
 #include "scan_walk.hpp"
 
 namespace clef {
-
-int device_cus();  // of the current device (gemm_f16.hip)
 namespace {
 
 constexpr int kC = 64;   // chunk length

@@ -312,7 +312,7 @@ static int launch_f32_split(const GemmParams& p, int epilogue, hipStream_t s) {
   return check_launch("gemm");
 }
 
-// Tile with the least rounds of 256 work-groups x time of a round (us at K =
+// Tile with the least rounds (a work-group per CU) x time of a round (us at K =
 // 2048, weights from HBM; one work-group per CU, and it walks K at the same
 // pace however many there are).  Where the lines fall (us, f32 MFMA kernel ->
 // now): N = 2048, K = 6144: M = 33 on 32 x 32 504 -> 57, M = 500 on 64 x 64
@@ -321,9 +321,10 @@ static int launch_f32_split(const GemmParams& p, int epilogue, hipStream_t s) {
 // 256 x 128 977 -> 552.
 static int gemm_f32_split_launch(const GemmParams& p, int epilogue, hipStream_t s) {
   const int n_eff = epilogue == 2 ? 2 * p.N : p.N;
+  const long cus = device_cus();
   auto cost = [&](int bm, int bn, double round) {
     const long tiles = (long)((p.M + bm - 1) / bm) * ((n_eff + bn - 1) / bn);
-    return (double)((tiles + 255) / 256) * round;
+    return (double)((tiles + cus - 1) / cus) * round;
   };
   const double c256 = cost(256, 128, 165), c128 = cost(128, 128, 100), c64 = cost(64, 64, 41), c32 = cost(32, 32, 19);
   if (c256 <= c128 && c256 <= c64 && c256 <= c32) return launch_f32_split<256, 128, 2, 4, 1, 1, true>(p, epilogue, s);

@@ -46,7 +46,4 @@ __device__ __forceinline__ void vm_wait_n(int n, std::integer_sequence<int, Ns..
 }
 __device__ __forceinline__ void vm_wait_n(int n) { vm_wait_n(n, std::make_integer_sequence<int, 40>{}); }
 
-// CUs of the current device (cached per device; gemm_f16.hip)
-int device_cus();
-
 }  // namespace clef
