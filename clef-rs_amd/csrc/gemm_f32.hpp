@@ -3,15 +3,19 @@
 // An f32 value is the exact sum of three bf16 values (8 + 8 + 8 significant
 // bits, the exponent range of f32), a bf16 product is exact in f32, and
 // v_mfma_f32_16x16x32_bf16 accumulates in f32 at 16 times the rate of the f32
-// MFMA.  x w = sum of nine such products; the six of relative size 2^-18 and
-// above are formed, the dropped three stay below 2^-26 of the term.  Each
+// MFMA.  Rounded to nearest, mid is at most 2^-8 of x and lo 2^-17, so of the
+// nine products in x w the three dropped ones (mid lo, lo mid, lo lo) reach
+// 2^-24 of the term at worst, as much as one f32 rounding, and 2^-26.5 in the
+// mean square over all significands.  The six others are formed.  Each
 // 32-deep step of K sums its products from zero, small ones first; steps are
 // added up in groups of four and the groups in a running sum, so the sum's
 // own magnitude is rounded once per 128 columns (the f32 MFMA kernel: once per
 // 32, after 16 roundings inside).  Against 64 bits, 2-norm, N(0,1) x N(0,0.02):
 // K = 64 0.58e-7 (f32 MFMA kernel 1.31e-7), K = 320 0.67e-7 (1.20e-7), K =
 // 2048 1.07e-7 (1.79e-7), K = 6144 1.68e-7 (2.74e-7); without the groups 1.60
-// and 2.69e-7 at the last two.
+// and 2.69e-7 at the last two.  With the significands that drop most in every
+// operand, both signs: K = 4 0.60e-7 (0.41e-7), K = 32 0.59e-7 (0.71e-7), K =
+// 2048 1.60e-7 (1.64e-7).
 // Outputs that the split does not hold (not finite, or where values below
 // 2^-100 matter) are formed on the f32 MFMA instead, at the end, their 16 x 16
 // blocks dealt to all waves.  At 2048 x 8192 x 2048 (f32 MFMA kernel 654 us,
@@ -188,7 +192,7 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_split(GemmParams p) {
 
   // 16 x 16 x 32 products, weights as the A operand (a lane's four results
   // are consecutive columns of one row).  Six products per block: all but
-  // mid*lo, lo*mid and lo*lo, at most 2^-26 of the term; the small ones first.
+  // mid*lo, lo*mid and lo*lo; the small ones first.
   // Each 32-deep step starts from zero, so the small products are summed
   // among themselves.
   const bool active = wave < VM * VN;

@@ -295,15 +295,41 @@ F32_SPLIT = [(1, 16, 4), (31, 33, 28), (33, 100, 196), (1, 2048, 6144), (65, 204
              (500, 8192, 96), (129, 4099, 64), (2048, 8192, 256), (1100, 9216, 100)]
 
 
+def _f32_split_bound(K):
+    return ((1 + 2.0 ** -10) + 2 * -(-K // 32) + -(-K // 128) + 1) * 2.0 ** -24
+
+
+@gpu
+@pytest.mark.parametrize("signs", [False, True])
+@pytest.mark.parametrize("M,N,K", [(33, 2048, 4), (33, 2048, 32), (300, 2000, 100), (2048, 8192, 64)])
+def test_gemm_f32_split_worst_significands(clef, M, N, K, signs):
+    """The significands whose split drops most (2^-24.01 of a product; found over all 2^23),
+    of one sign, where the dropped parts add up, and of both."""
+    bits = torch.tensor([0x3f807fc0, 0x3f808040, 0x3f807f40, 0x3f8080c0], dtype=torch.int32, device="cuda")
+    worst = bits.view(torch.float32)
+    gen = torch.Generator(device="cuda").manual_seed(45)
+
+    def draw(*shape):
+        v = worst[torch.randint(4, shape, generator=gen, device="cuda")]
+        v = v * 2.0 ** torch.randint(-3, 4, shape, generator=gen, device="cuda").float()
+        return v * (1 - 2 * torch.randint(2, shape, generator=gen, device="cuda").float()) if signs else v
+
+    x, w = draw(M, K), draw(N, K)
+    y = clef.gemm(x, w).double()
+    err = (y - x.double() @ w.double().T).abs()
+    assert (err <= _f32_split_bound(K) * (x.double().abs() @ w.double().abs().T)).all()
+
+
 @gpu
 @pytest.mark.parametrize("M,N,K", F32_SPLIT)
 def test_gemm_f32_split_tiles(clef, M, N, K):
-    """The split forms each product to 2^-26 of the term and rounds a sum at
-    most twice per 32 columns: |err| <= (2^-25 + (6 + K / 16) 2^-24) sum|x w|."""
+    """The split drops at most (1 + 2^-10) 2^-24 of a term (mid lo + lo mid + lo lo, mid <=
+    2^-8 and lo <= 2^-17 of the value) and rounds a sum twice per 32 columns, once more per
+    128 and at the end: |err| <= ((1 + 2^-10) + 2 ceil(K / 32) + ceil(K / 128) + 1) 2^-24 sum|x w|."""
     x, w = _inputs(31, M, N, K, torch.float32)
     _, u = _inputs(32, 1, N, K, torch.float32)
     ref, scale = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
-    bound = (2.0 ** -25 + (6 + K / 16) * 2.0 ** -24) * scale
+    bound = _f32_split_bound(K) * scale
     y = clef.gemm(x, w)
     assert ((y.double() - ref).abs() <= bound).all()
     # in the 2-norm the error of a random sum is far smaller: below that of the
