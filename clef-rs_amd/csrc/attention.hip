@@ -32,9 +32,9 @@ constexpr int attn_lds_bytes() {
   return (64 * (D + EPF) + D * (64 + EPF) + 4 * 16 * (64 + EPF)) * (int)sizeof(T);
 }
 
-// 64 query rows of one head, by the first four waves of a work-group (any
-// others only keep its barriers).
-template <class T, int D>
+// 64 query rows of one head, by the first four waves of a work-group of NT
+// threads (any others help to move the keys and values).
+template <class T, int D, int NT>
 __device__ __forceinline__ void attn_body(const AttnParams& p, char* smem) {
   constexpr int BQ = 64, BKEY = 64;
   constexpr int EPF = 16 / sizeof(T);
@@ -52,7 +52,7 @@ __device__ __forceinline__ void attn_body(const AttnParams& p, char* smem) {
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const bool on = wave < 4;
+  const bool on = NT == 256 || wave < 4;
   const int col = lane & 15, grp = lane >> 4;
   const int qtiles = (p.qn + BQ - 1) / BQ;
   const int h = blockIdx.x % p.heads;
@@ -91,20 +91,20 @@ __device__ __forceinline__ void attn_body(const AttnParams& p, char* smem) {
   // K [64][D] and V^T [D][64] of a key tile: loaded into registers during the
   // previous tile's products, written to LDS after them
   constexpr int KV_PER_ROW = D / EPF, V_PER_ROW = BKEY / EPF;
-  constexpr int NKL = BKEY * KV_PER_ROW / 256, NVL = D * V_PER_ROW / 256;  // vectors per thread
-  static_assert(BKEY * KV_PER_ROW % 256 == 0 && D * V_PER_ROW % 256 == 0, "whole passes");
+  constexpr int NKL = BKEY * KV_PER_ROW / NT, NVL = D * V_PER_ROW / NT;  // vectors per thread
+  static_assert(BKEY * KV_PER_ROW % NT == 0 && D * V_PER_ROW % NT == 0, "whole passes");
   vec kreg[NKL], vreg[NVL];
   auto load_tile = [&](int j0) {
 #pragma unroll
     for (int u = 0; u < NKL; ++u) {
-      const int v = tid + 256 * u;
+      const int v = tid + NT * u;
       const int r = v / KV_PER_ROW, c = (v % KV_PER_ROW) * EPF;
       const int key = min(j0 + r, p.kn - 1);
       kreg[u] = c < d ? *reinterpret_cast<const vec*>(K + (int64_t)key * d + c) : vec{};
     }
 #pragma unroll
     for (int u = 0; u < NVL; ++u) {
-      const int v = tid + 256 * u;
+      const int v = tid + NT * u;
       const int r = v / V_PER_ROW, c = (v % V_PER_ROW) * EPF;
       const int key = min(j0 + c, p.ldv - EPF);
       vreg[u] = r < d ? *reinterpret_cast<const vec*>(V + (int64_t)r * p.ldv + key) : vec{};
@@ -113,13 +113,13 @@ __device__ __forceinline__ void attn_body(const AttnParams& p, char* smem) {
   auto store_tile = [&](int j0) {
 #pragma unroll
     for (int u = 0; u < NKL; ++u) {
-      const int v = tid + 256 * u;
+      const int v = tid + NT * u;
       const int r = v / KV_PER_ROW, c = (v % KV_PER_ROW) * EPF;
       *reinterpret_cast<vec*>(&sK[r * LDK + c]) = kreg[u];
     }
 #pragma unroll
     for (int u = 0; u < NVL; ++u) {
-      const int v = tid + 256 * u;
+      const int v = tid + NT * u;
       const int r = v / V_PER_ROW, c = (v % V_PER_ROW) * EPF;
       const int key = min(j0 + c, p.ldv - EPF);
       vec vv = vreg[u];
@@ -129,19 +129,20 @@ __device__ __forceinline__ void attn_body(const AttnParams& p, char* smem) {
       *reinterpret_cast<vec*>(&sV[r * LDV + c]) = vv;
     }
   };
-  if (on) {
-    load_tile(0);
-    store_tile(0);
-  }
+  load_tile(0);
+  store_tile(0);
   lds_barrier();
   for (int j0 = 0; j0 < key_end; j0 += BKEY) {
     const bool more = j0 + BKEY < key_end;  // uniform over the work-group
+    if (more) load_tile(j0 + BKEY);
     if (!on) {
       lds_barrier();
-      if (more) lds_barrier();
+      if (more) {
+        store_tile(j0 + BKEY);
+        lds_barrier();
+      }
       continue;
     }
-    if (more) load_tile(j0 + BKEY);
 
     // ---- S = Q K^T for 16 rows x 64 keys
     float4_t S[4];
@@ -239,7 +240,7 @@ __device__ __forceinline__ void attn_body(const AttnParams& p, char* smem) {
 template <class T, int D>
 __global__ __launch_bounds__(256) void attn_kernel(AttnParams p) {
   __shared__ __attribute__((aligned(16))) char smem[attn_lds_bytes<T, D>()];
-  attn_body<T, D>(p, smem);
+  attn_body<T, D, 256>(p, smem);
 }
 
 #include "attention_f32.hpp"

@@ -347,7 +347,7 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split(AttnParams p) {
   lds_barrier();
   if (*redo == 0) return;
   lds_barrier();  // the flag's place is attn_body's from here on
-  attn_body<float, D>(p, smem);
+  attn_body<float, D, 512>(p, smem);
 }
 
 // d of a whole tile, 16-byte aligned rows, a head's keys and values within 31-bit byte offsets
