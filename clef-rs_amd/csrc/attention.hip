@@ -33,9 +33,10 @@ constexpr int attn_lds_bytes() {
 }
 
 // 64 query rows of one head, by the first four waves of a work-group of NT
-// threads (any others help to move the keys and values).
+// threads (any others help to move the keys and values); stores the rows of the
+// mask `rows`.
 template <class T, int D, int NT>
-__device__ __forceinline__ void attn_body(const AttnParams& p, char* smem) {
+__device__ __forceinline__ void attn_body(const AttnParams& p, char* smem, uint64_t rows) {
   constexpr int BQ = 64, BKEY = 64;
   constexpr int EPF = 16 / sizeof(T);
   constexpr int KB = Mma<T>::kBlock;
@@ -219,7 +220,7 @@ __device__ __forceinline__ void attn_body(const AttnParams& p, char* smem) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int row = q0 + wave * 16 + grp * 4 + i;
-    if (row >= p.qn) continue;
+    if (row >= p.qn || !(rows >> (row - q0) & 1)) continue;
     const float inv = 1.0f / l[i];
 #pragma unroll
     for (int nt = 0; nt < NDT; ++nt) {
@@ -240,7 +241,7 @@ __device__ __forceinline__ void attn_body(const AttnParams& p, char* smem) {
 template <class T, int D>
 __global__ __launch_bounds__(256) void attn_kernel(AttnParams p) {
   __shared__ __attribute__((aligned(16))) char smem[attn_lds_bytes<T, D>()];
-  attn_body<T, D, 256>(p, smem);
+  attn_body<T, D, 256>(p, smem, ~uint64_t(0));
 }
 
 #include "attention_f32.hpp"

@@ -20,8 +20,16 @@
 // these are the 8 consecutive keys of its B fragment of O^T = V^T P^T, and P
 // goes from the softmax into the products without passing LDS.
 //
-// A work-group that met values which the split does not hold (infinities, NaN,
-// below 2^-100) runs attn_body instead, at the end.
+// The split errs by up to 2^-124 for values below 2^-100.  With keys and queries
+// below 2^90 that moves a score by less than 2^-26; it moves an output of 2^-97
+// or more by less than 2^-27 of itself.  (Probabilities below 2^-100 of the row's
+// largest are held to 2^-124 too.)  A query is formed again by attn_body, at the
+// end, if it or a key it sees is larger, or if one of its outputs is not finite
+// or, with a value below 2^-100 in sight, smaller: that follows from the query
+// and what it sees, not from those that share its tile.  777 queries behind 256
+// keys, 16 heads x 256 (us; f32 MFMA kernel 227, here 124): a value below 2^-100
+// in one key or value row 124; a column of V wholly below 377, an infinity that
+// half of the queries see 366, one NaN query 155.
 //
 // What bounds it: LDS.  A fragment of three planes feeds six products, so with
 // 16 queries per wave a key tile reads as many LDS cycles as it multiplies,
@@ -51,7 +59,9 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split(AttnParams p) {
   static_assert(BK * CPR % 256 == 0, "whole chunks per thread");
   static_assert(kLds <= 160 * 1024, "LDS");
   __shared__ __attribute__((aligned(16))) char smem[kLds];
-  int* const redo = reinterpret_cast<int*>(smem + kTiles + kQ) - 1;  // once Q is no longer read
+  // once Q is no longer read: the first large key, the first with a tiny value,
+  // and the rows to form again, 16 per wave of group 0
+  int* const flags = reinterpret_cast<int*>(smem + kTiles + kQ) - 6;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -69,22 +79,33 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split(AttnParams p) {
   const float* K = static_cast<const float*>(p.k) + (int64_t)kvh * p.ldk * D;
   const float* V = static_cast<const float*>(p.vt) + (int64_t)kvh * D * p.ldv;
 
-  uint32_t smallest = 0xffffffffu;  // of |x| > 0, as 2 * bits - 1
-  auto split = [&](const float4_t& a, const float4_t& b, bf16x8* pl) {
+  constexpr float kSmallOut = 0x1p-97f;
+  constexpr uint32_t kLarge = 217u << 24, kTiny = 27u << 24;  // 2 * bits of 2^90 and 2^-100
+  auto largest = [](uint32_t m, const float4_t& a, const float4_t& b) {  // of 2 * bits
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      smallest = min(smallest, 2u * __float_as_uint(a[e]) - 1u);
-      smallest = min(smallest, 2u * __float_as_uint(b[e]) - 1u);
-    }
-    split8(a, b, pl[0], pl[1], pl[2]);
+    for (int e = 0; e < 4; ++e) m = max(max(m, 2u * __float_as_uint(a[e])), 2u * __float_as_uint(b[e]));
+    return m;
   };
+  auto least = [](uint32_t m, const float4_t& a, const float4_t& b) {  // of 2 * bits - 1 (0 last)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) m = min(min(m, 2u * __float_as_uint(a[e]) - 1u), 2u * __float_as_uint(b[e]) - 1u);
+    return m;
+  };
+  constexpr int kNone = 0x7fffffff;
+  auto wave_least = [](int x) {
+    for (int o = 1; o < 64; o <<= 1) x = min(x, __shfl_xor(x, o, 64));
+    return __builtin_amdgcn_readfirstlane(x);
+  };
+  int first_large = kNone, first_tiny = kNone;  // keys, of those that this wave split
 
   // Q fragments (B operand): d = 32 kb + 8 g .. + 7 of query n; the mid and lo
   // planes, half of the products, wait in LDS (both groups use the same rows;
   // in registers they spill, and a reload waits for the prefetch as well)
   bf16x8 qf[NKB];
   bf16x8* const qml = reinterpret_cast<bf16x8*>(smem + kTiles) + wq * NKB * 128 + lane;
+  uint64_t large_q;  // by lane
   {
+    uint32_t q_large = 0;
     const float* row = Q + (int64_t)min(q0 + 16 * wq + n, p.qn - 1) * D + 8 * g;
     float4_t raw[NKB][2];
 #pragma unroll
@@ -94,13 +115,15 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split(AttnParams p) {
 #pragma unroll
     for (int kb = 0; kb < NKB; ++kb) {
       bf16x8 pl[3];
-      split(raw[kb][0], raw[kb][1], pl);
+      split8(raw[kb][0], raw[kb][1], pl[0], pl[1], pl[2]);
+      q_large = largest(q_large, raw[kb][0], raw[kb][1]);
       qf[kb] = pl[0];
       if (grp == 0) {  // published by the first phase's barrier
         qml[kb * 128] = pl[1];
         qml[kb * 128 + 64] = pl[2];
       }
     }
+    large_q = __ballot(q_large >= kLarge);
   }
 
   // one register set holds the next operand to be split: V of a tile is
@@ -144,16 +167,26 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split(AttnParams p) {
 #pragma unroll
     for (int s = 0; s < 3; ++s) *reinterpret_cast<bf16x8*>(dst + s * kPlane) = pl[s];
   };
-  auto put_k = [&] {
+  auto put_k = [&](int j0) {
+    uint32_t m = 0;
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
       const int ci = i * 256 + gt, r = ci / CPR, c = ci % CPR;
       bf16x8 pl[3];
-      split(ld[i][0], ld[i][1], pl);
+      split8(ld[i][0], ld[i][1], pl[0], pl[1], pl[2]);
+      m = largest(m, ld[i][0], ld[i][1]);
       store(planes + r * D + ((c ^ kswizzle(r)) << 3), pl);
+    }
+    if (__ballot(m >= kLarge) != 0) {
+      int key = kNone;
+#pragma unroll
+      for (int i = CH - 1; i >= 0; --i)
+        if (largest(0, ld[i][0], ld[i][1]) >= kLarge) key = j0 + (i * 256 + gt) / CPR;
+      first_large = min(first_large, wave_least(key));
     }
   };
   auto put_v = [&](int j0) {
+    uint32_t m = 0xffffffffu;
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
       const int ci = i * 256 + gt, r = ci >> 2, c = ci & 3, key = j0 + 8 * c;
@@ -165,9 +198,22 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split(AttnParams p) {
           if (key + 4 + e >= p.kn) b[e] = 0.0f;
         }
       }
+      m = least(m, a, b);
       bf16x8 pl[3];
-      split(a, b, pl);
+      split8(a, b, pl[0], pl[1], pl[2]);
       store(planes + r * 32 + ((c ^ ((r >> 2) & 3)) << 3), pl);
+    }
+    if (__ballot(m < kTiny - 1u) != 0) {
+      int first = kNone;
+#pragma unroll
+      for (int e = 7; e >= 0; --e) {
+        const int key = j0 + vc0 + e;
+        bool tiny = false;
+#pragma unroll
+        for (int i = 0; i < CH; ++i) tiny |= 2u * __float_as_uint(ld[i][e >> 2][e & 3]) - 1u < kTiny - 1u;
+        if (tiny && key < p.kn) first = key;
+      }
+      first_tiny = min(first_tiny, wave_least(first));
     }
   };
 
@@ -282,7 +328,7 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split(AttnParams p) {
     const int j0 = first + st * 2 * BK;
     const bool here = j0 < key_end;
     if (here) {
-      put_k();
+      put_k(j0);
       load_v(j0);
     }
     lds_barrier();
@@ -307,34 +353,57 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split(AttnParams p) {
     ml[0] = m;
     ml[1] = l;
   }
-  if (tid == 0) *redo = 0;
+  if (tid < 2) flags[tid] = kNone;
+  const int row = q0 + 16 * wq + n, rowc = min(row, p.qn - 1);
+  float4_t gv[NDT];  // requested here: behind the barriers they are in
+  if (grp == 0) {
+    const float* gate = static_cast<const float*>(p.gate) + (int64_t)rowc * p.ldg + (int64_t)h * p.hsg + 4 * g;
+#pragma unroll
+    for (int t = 0; t < NDT; ++t) {
+      if (p.vec_io) {
+        gv[t] = *reinterpret_cast<const float4_t*>(gate + 16 * t);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) gv[t][i] = gate[16 * t + i];
+      }
+    }
+  }
   lds_barrier();
-  if (smallest < (27u << 24) - 1u) *redo = 1;
+  if (lane == 0) {
+    if (first_large != kNone) atomicMin(&flags[0], first_large);
+    if (first_tiny != kNone) atomicMin(&flags[1], first_tiny);
+  }
+  lds_barrier();
   if (grp == 0) {
     const float m1 = ml[0], mn = fmaxf(m, m1);
     const float a0 = expf(m - mn), a1 = m1 == -INFINITY ? 0.0f : expf(m1 - mn);  // (key 0 is in group 0: m is not -inf)
     const float inv = 1.0f / (l * a0 + ml[1] * a1);
-    const int row = q0 + 16 * wq + n, rowc = min(row, p.qn - 1);
-    const float* gate = static_cast<const float*>(p.gate) + (int64_t)rowc * p.ldg + (int64_t)h * p.hsg + 4 * g;
-    float* y = static_cast<float*>(p.y) + (int64_t)rowc * p.ldy + (int64_t)h * D + 4 * g;
-    bool odd = false;
+    const bool tiny = flags[1] <= lim;
+    bool odd = flags[0] <= lim || (large_q >> lane & 1) != 0;
 #pragma unroll
     for (int t = 0; t < NDT; ++t) {
       const float4_t o1 = *reinterpret_cast<const float4_t*>(mo + t * (4 * 64 * 4));
-      float4_t o, gv;
-      if (p.vec_io) {
-        gv = *reinterpret_cast<const float4_t*>(gate + 16 * t);
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) gv[i] = gate[16 * t + i];
-      }
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float a = (O[t][i] * a0 + o1[i] * a1) * inv;
-        odd |= !(fabsf(a) < INFINITY);
-        o[i] = a * (1.0f / (1.0f + expf(-gv[i])));
+        odd |= !(fabsf(a) < INFINITY) || (tiny && fabsf(a) < kSmallOut);
+        O[t][i] = a;
       }
-      if (row >= p.qn) continue;
+    }
+    // a query's outputs are spread over four lanes
+    uint64_t rows = __ballot(odd);
+    rows |= rows >> 32;
+    rows = (rows | rows >> 16) & 0xffff;
+    if (lane == 0) flags[2 + wq] = static_cast<int>(rows);
+    float* y = static_cast<float*>(p.y) + (int64_t)rowc * p.ldy + (int64_t)h * D + 4 * g;
+    // (rows to form again are not stored here: a caller may gate in place)
+    const bool here = row < p.qn && !(rows >> n & 1);
+#pragma unroll
+    for (int t = 0; t < NDT; ++t) {
+      float4_t o;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = O[t][i] * (1.0f / (1.0f + expf(-gv[t][i])));
+      if (!here) continue;
       if (p.vec_io) {
         *reinterpret_cast<float4_t*>(y + 16 * t) = o;
       } else {
@@ -342,12 +411,15 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split(AttnParams p) {
         for (int i = 0; i < 4; ++i) y[16 * t + i] = o[i];
       }
     }
-    if (odd) *redo = 1;
   }
   lds_barrier();
-  if (*redo == 0) return;
-  lds_barrier();  // the flag's place is attn_body's from here on
-  attn_body<float, D, 512>(p, smem);
+  uint64_t again = 0;
+#pragma unroll
+  for (int w = 0; w < 4; ++w)
+    again |= (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane(flags[2 + w]) << (16 * w);
+  if (again == 0) return;
+  lds_barrier();  // the flags' place is attn_body's from here on
+  attn_body<float, D, 512>(p, smem, again);
 }
 
 // d of a whole tile, 16-byte aligned rows, a head's keys and values within 31-bit byte offsets

@@ -465,3 +465,66 @@ def test_attention_f32_values_the_split_does_not_hold(clef):
     assert (y[:, 7].double() - ref[:, 7]).norm() <= 1e-5 * ref[:, 7].norm()
     assert (y[:, 8] == 0).all()
     assert torch.allclose(y[:, 9:].double(), ref[:, 9:], rtol=1e-4, atol=1e-5)
+
+
+@gpu
+@pytest.mark.parametrize("heads,kvh,d", [(4, 2, 256), (3, 1, 128), (2, 2, 64)])
+def test_attention_f32_queries_do_not_depend_on_their_neighbours(clef, heads, kvh, d):
+    """Large, tiny and non-finite elements change the queries that see them and no other, and a
+    query's bits do not depend on which others share its 64-query tile."""
+    qn, kn = 200, 230
+    gen = torch.Generator(device="cuda").manual_seed(73)
+    rnd = lambda *s: torch.randn(s, generator=gen, device="cuda")
+    q, k, v, gate = rnd(heads, qn, d), rnd(kvh, kn, d), rnd(kvh, kn, d), rnd(qn, heads, d)
+
+    def run(q, k, v, gate):
+        vt = torch.zeros((kvh, d, 232), device="cuda")
+        vt[:, :, :kn] = v.transpose(1, 2)
+        return clef.attention_gated(q.contiguous(), k, vt, gate, kn=kn)
+
+    plain = run(q, k, v, gate)
+    off = kn - qn
+    for name, key in (("tiny key", 100), ("tiny value", 100), ("large key", 101), ("large value", 159),
+                      ("infinite key", 224), ("nan query", 70), ("large query", 71)):
+        q1, k1, v1 = q.clone(), k.clone(), v.clone()
+        if name == "tiny key":
+            k1[0, key, 3] = 1e-36
+        elif name == "tiny value":
+            v1[0, key, 3] = -1e-36
+        elif name == "large key":
+            k1[0, key, 3] = 3e27
+        elif name == "large value":
+            v1[0, key, 3] = 1e9
+        elif name == "infinite key":
+            k1[0, key, 3] = float("inf")
+        elif name == "nan query":
+            q1[1, key, 3] = float("nan")
+        elif name == "large query":
+            q1[1, key, 3] = 2e27
+        y = run(q1, k1, v1, gate)
+        first = key if "query" in name else key - off  # the first query it reaches
+        assert torch.equal(y[:first], plain[:first]), name
+        if "query" in name:
+            assert torch.equal(y[first + 1:], plain[first + 1:]), name
+        # the same queries at another place in their tiles
+        assert torch.equal(torch.nan_to_num(run(q1[:, 10:], k1, v1, gate[10:]), nan=1e30),
+                           torch.nan_to_num(y[10:], nan=1e30)), name
+
+
+@gpu
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_attention_f32_gates_in_place(clef, d):
+    """y may be the gate's own memory, also where queries are formed again."""
+    heads, kvh, qn = 4, 2, 150
+    gen = torch.Generator(device="cuda").manual_seed(74)
+    rnd = lambda *s: torch.randn(s, generator=gen, device="cuda")
+    q, k, vt, gate = rnd(heads, qn, d), rnd(kvh, qn, d), rnd(kvh, d, 152), rnd(qn, heads * d)
+    vt[:, 5] *= 1e-35
+    q[1, 77] = float("nan")
+    y = clef.attention_gated(q, k, vt, gate.view(qn, heads, d), kn=qn)
+    buf = gate.clone()
+    rc = clef.lib().clef_attention_gated(q.data_ptr(), qn, k.data_ptr(), qn, vt.data_ptr(), 152, 0, heads, kvh, qn, qn,
+                                         d, buf.data_ptr(), heads * d, d, buf.data_ptr(), heads * d,
+                                         torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    assert torch.equal(torch.nan_to_num(buf, nan=1e30), torch.nan_to_num(y, nan=1e30))
