@@ -222,17 +222,20 @@ def test_silu_mul_rejects_bad_arguments(clef):
 
 # launches on small tiles (32 x 16, 64 x 32, 64 x 64, 128 x 64): one row, tile
 # edges and remainders in rows and columns, odd row pitches, one K stage,
-# partial stages (K = 320, 192), a request-sized call of each projection
-SMALL = [(1, 2048, 6144), (33, 2048, 6144), (31, 100, 64), (64, 1000, 320), (65, 73, 192), (200, 2048, 4096),
-         (129, 2047, 1024), (1, 12288, 2048), (37, 12288, 2048), (100, 12288, 2048), (300, 2048, 2048),
-         (500, 2000, 512), (1000, 2048, 6144)]
+# partial stages (K = 320, 192), a request-sized call of each projection.  With
+# 12288 rows N = 1000 and more takes 128- or 256-row tiles of the other kernels,
+# N = 100 and 73 still 128 x 64 (their columns' edges; the order of their sums is
+# that of N = 1000 with the same K)
+SMALL = [(1, 2048, 6144), (33, 2048, 6144), (31, 100, 64), (31, 1000, 64), (64, 1000, 320), (65, 73, 192),
+         (65, 1000, 192), (200, 2048, 4096), (129, 2047, 1024), (1, 12288, 2048), (37, 12288, 2048),
+         (100, 12288, 2048), (300, 2048, 2048), (500, 2000, 512), (1000, 2048, 6144)]
 
 
 @gpu
 @pytest.mark.parametrize("M,N,K", SMALL)
 def test_gemm_small_tiles(clef, M, N, K):
     """Each epilogue against the reference, and equal bit for bit to the same
-    rows of a call with enough rows for the large tiles (one summation order)."""
+    rows of a call of 12288 rows (one summation order on all tiles)."""
     x, w = _inputs(21, M, N, K, torch.float16)
     _, u = _inputs(22, 1, N, K, torch.float16)
     rows = 4096 * 3
