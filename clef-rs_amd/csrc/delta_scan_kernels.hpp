@@ -265,8 +265,8 @@ constexpr int kPW = 8;  // waves of a scan_prepare work-group
 // on one wave, reads of the inversion requested ahead and its off-diagonal
 // blocks without barriers shortened it: the first three took a work-group's
 // 31800 cycles (f16, two heads; these steps 17400) to 27500 (12200).
-// 16 / 32 heads x 128, us, f16 and f32: T = 4096 37.5 -> 33.8, 88.7 -> 82.3;
-// T = 1000 18.0 -> 16.2, 24.6 -> 22.8; T = 100 10.8 -> 8.8, 15.3 -> 14.4.
+// 16 / 32 heads x 128, us, f16 and f32: T = 4096 37.5 -> 33.8, 88.7 -> 77.3;
+// T = 1000 18.0 -> 16.2, 24.6 -> 21.9; T = 100 10.8 -> 9.5, 15.3 -> 14.0.
 //
 // Two work-groups per CU (16 waves, 128 registers each) where the LDS holds
 // two; f32 products with 128-wide keys need more LDS than half a CU.
@@ -620,11 +620,12 @@ __global__ __launch_bounds__(64 * kPW, (sizeof(CT) == 4 && DK > 64) ? 2 : 4) voi
 //
 // Wave 0 runs the recurrence; loader waves fill a ring of LDS slots, D0 - 1
 // chunks ahead, with global->LDS DMA (f16: wave 1 the chunk's raw key rows,
-// wave 2 its U blocks and row scalars; f32: wave 1 both); output waves form
-// the outputs of the previous chunk (f16: four waves of one 16-row tile, f32:
-// two of two) from the S and Y that wave 0 hands over in LDS and from query
-// rows and N blocks they load into registers a few chunks ahead.  One
-// barrier per chunk.
+// wave 2 its U blocks and row scalars; f32: one wave both); output waves form
+// the outputs of the previous chunk (four waves of one 16-row tile; two of two
+// where f32 has one recurrence wave) from the S and Y that the recurrence hands
+// over in LDS and from query rows and N blocks they load into registers a few
+// chunks ahead.  One barrier per chunk.  (f32 products: up to four recurrence
+// waves share wave 0's work, see Carry.)
 //
 // Norms as row factors: with a_r = 1/|k_r| and b_r = qscale/|q_r|,
 //   e^gam (K^ S) = diag(a e^gam) (K S),   e^gam (Q^ S) = diag(b e^gam) (Q S),
@@ -732,9 +733,10 @@ __device__ __forceinline__ void lds_wait_all(const unsigned* flags, int n, unsig
 
 // Token span of chunk c of the work-group's sequence: a sequence's chunks
 // are 64-token steps from its first token (the chunk table holds exactly
-// these spans), so no table is read on the carry's paths; a lookup there
+// these spans), so a walk of one sequence reads no table; a vector lookup
 // makes each step wait for it, and in-order vmcnt then drains every load
-// in flight behind it.
+// in flight behind it.  (A walk of all sequences reads the table through the
+// scalar cache, chunk_entry.)
 struct CarryCtx {
   int h, hk, j0, jc;
   bool col_ok;
@@ -1421,7 +1423,7 @@ int launch_dk(const ScanParams& p, hipStream_t stream) {
   // one (the Gram tiles are formed again).  16 / 32 heads x 128, us: T = 100
   // f16 14.2 -> 10.8, f32 20.5 -> 15.3; T = 400 16.0 -> 12.6, 23.5 -> 18.4; at
   // T = 600 (320 work-groups) 16.5 -> 16.0, f32 24.0 -> 30.2 (the head's steps
-  // have since become shorter: T = 400 now 11.0 and 17.7, 600 15.8 and 22.8).
+  // have since become shorter: T = 400 now 11.3 and 17.0).
   const int vsplit = (int64_t)p.nchunks * p.Hv <= device_cus() ? p.Hv / p.Hk : 1;
   hipLaunchKernelGGL((scan_prepare<CT, IT, DK>), dim3(p.nchunks, p.Hk, vsplit), dim3(64 * kPW), 0, stream, p);
   int rc = check_launch("scan_prepare");

@@ -114,8 +114,8 @@ __host__ __device__ inline bool chunk_last(int w) { return (w >> 7 & 1) != 0; }
 __host__ __device__ inline int chunk_seq(int w) { return w >> 8; }
 
 // Scan, step 6: per sequence its chunks (ctab: first token, chunk_word) and its
-// entry in stab ({sequence, first chunk, chunks, 0}) at its
-// rank by chunk count (most first, ties in sequence order).
+// entry in stab ({sequence, first chunk, chunks, 0}) at its rank by chunk count
+// (most first, ties in sequence order).
 __host__ __device__ inline void rg_scan_6(const Ragged& g, int tid, int chunk, int* ctab, int* stab) {
   int s0, s1;
   rg_range(tid, g.nseq, s0, s1);
