@@ -177,7 +177,7 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split(AttnParams p) {
       m = largest(m, ld[i][0], ld[i][1]);
       store(planes + r * D + ((c ^ kswizzle(r)) << 3), pl);
     }
-    if (__ballot(m >= kLarge) != 0) {
+    if (__builtin_expect(__ballot(m >= kLarge) != 0, 0)) {
       int key = kNone;
 #pragma unroll
       for (int i = CH - 1; i >= 0; --i)
@@ -203,7 +203,7 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split(AttnParams p) {
       split8(a, b, pl[0], pl[1], pl[2]);
       store(planes + r * 32 + ((c ^ ((r >> 2) & 3)) << 3), pl);
     }
-    if (__ballot(m < kTiny - 1u) != 0) {
+    if (__builtin_expect(__ballot(m < kTiny - 1u) != 0, 0)) {
       int first = kNone;
 #pragma unroll
       for (int e = 7; e >= 0; --e) {

@@ -94,7 +94,7 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_split(GemmParams p) {
   // of [x rows | weight rows], formed only if the tile met a value below 2^-100:
   // K 2^-97 if the row holds one, else 0; its largest magnitude
   __shared__ float row_tiny[ROWS], row_max[ROWS];
-  __shared__ int any_tiny, any_redo;
+  __shared__ int any_tiny, any_odd;  // a value below 2^-100, or that or an output that is not finite
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -248,7 +248,7 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_split(GemmParams p) {
     }
   };
 
-  if (tid == 0) any_tiny = any_redo = 0;
+  if (tid == 0) any_tiny = any_odd = 0;
   load(0, 0);
   if (D == 2 && nst > 1) load(1, 1);
   split(0, 0);
@@ -349,38 +349,17 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_split(GemmParams p) {
   // err by less than 2^-27), is formed again on f32 products.  That follows
   // from the row, the column and the result alone, so a row's bits do not
   // depend on what shares its tile.
-  if (smallest < kTiny) any_tiny = 1;
+  const bool small = smallest < kTiny;
+  float4_t z = {0.f, 0.f, 0.f, 0.f};  // NaN once something is not finite
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) z[e] = fmaf(tot[i][j][e], 0.0f, z[e]);
+  if (small) any_tiny = 1;
+  if (small || z[0] + z[1] + z[2] + z[3] != 0.0f) any_odd = 1;
   lds_barrier();
-  const bool tiny = __builtin_amdgcn_readfirstlane(any_tiny) != 0;
-  if (tiny) {
-    // the rows once more, four of them a wave at a time
-    const int rl = lane >> 4, cl = 4 * (lane & 15);
-    for (int row = 4 * wave + rl; row < ROWS; row += 32) {
-      const bool is_x = row < BM;
-      const int rb = row - BM;
-      const float* op = is_x ? X : EPI == 2 && (rb & 16) ? W2 : W;
-      const int r = is_x ? min(m0 + row, p.M - 1) : min(n0 + (EPI == 2 ? (rb >> 5) * 16 + (rb & 15) : rb), p.N - 1);
-      const float* src = op + (int64_t)r * (is_x ? p.ldx : p.ldw);
-      float m = 0.0f;
-      uint32_t least = 0xffffffffu;
-      for (int k0 = 0; k0 < p.K; k0 += 512) {
-        float4_t v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = *reinterpret_cast<const float4_t*>(src + min(k0 + 64 * u + cl, p.K - 4));
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            m = fmaxf(m, fabsf(v[u][e]));
-            least = min(least, 2u * __float_as_uint(v[u][e]) - 1u);
-          }
-      }
-      m = lane_max<16>(m);
-      const float t = lane_max<16>(least < kTiny ? static_cast<float>(p.K) * 0x1p-97f : 0.0f);
-      if (cl == 0) row_max[row] = m, row_tiny[row] = t;
-    }
-    lds_barrier();
-  }
 
   const int esz = (EPI == 1 || p.dtype_out != 1) ? 4 : 2;
   const bool yvec = ((reinterpret_cast<uintptr_t>(p.y) | (uintptr_t)(p.ldy * esz)) & (4 * esz - 1)) == 0;
@@ -423,47 +402,71 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_split(GemmParams p) {
       store_row4(p, r, c, v, whole, skip);
     }
   };
-  bool odd_any = tiny;
+  if (__builtin_expect(any_odd == 0, 1)) {
+    if (active)
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
+      for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
+        for (int j = 0; j < TO; ++j)
+          finish(orow(wave, i), ocol(wave, j), tot[i][EPI == 2 ? 2 * j : j], tot[i][EPI == 2 ? 2 * j + 1 : j], 0);
+    return;
+  }
+  const bool tiny = __builtin_amdgcn_readfirstlane(any_tiny) != 0;
+  if (tiny) {
+    // the rows once more, four of them a wave at a time
+    const int rl = lane >> 4, cl = 4 * (lane & 15);
+    for (int row = 4 * wave + rl; row < ROWS; row += 32) {
+      const bool is_x = row < BM;
+      const int rb = row - BM;
+      const float* op = is_x ? X : EPI == 2 && (rb & 16) ? W2 : W;
+      const int r = is_x ? min(m0 + row, p.M - 1) : min(n0 + (EPI == 2 ? (rb >> 5) * 16 + (rb & 15) : rb), p.N - 1);
+      const float* src = op + (int64_t)r * (is_x ? p.ldx : p.ldw);
+      float m = 0.0f;
+      uint32_t least = 0xffffffffu;
+      for (int k0 = 0; k0 < p.K; k0 += 512) {
+        float4_t v[8];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) odd_any |= !(fabsf(tot[i][j][e]) < __builtin_inff());
+        for (int u = 0; u < 8; ++u) v[u] = *reinterpret_cast<const float4_t*>(src + min(k0 + 64 * u + cl, p.K - 4));
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            m = fmaxf(m, fabsf(v[u][e]));
+            least = min(least, 2u * __float_as_uint(v[u][e]) - 1u);
+          }
+      }
+      m = lane_max<16>(m);
+      const float t = lane_max<16>(least < kTiny ? static_cast<float>(p.K) * 0x1p-97f : 0.0f);
+      if (cl == 0) row_max[row] = m, row_tiny[row] = t;
+    }
+    lds_barrier();
+  }
   uint64_t redo = 0;  // bit 4 (i TO + j) + e
-  if (active && __ballot(odd_any) != 0) {
+  if (active) {
     const int xr = wm * WM + r16, wr = BM + wn * WN + 4 * c16;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TO; ++j) {
         const int j0 = EPI == 2 ? 2 * j : j, j1 = EPI == 2 ? 2 * j + 1 : j;
-        uint32_t odd = 0;
+        uint32_t again = 0;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          auto again = [&](int jj) {
+          auto is = [&](int jj) {
             const float a = fabsf(tot[i][jj][e]);
             if (!tiny) return !(a < __builtin_inff());
             const int x = xr + 16 * i, w = wr + 16 * jj + e;
             return !(a < __builtin_inff()) || a < row_tiny[x] * row_max[w] + row_tiny[w] * row_max[x];
           };
-          odd |= (again(j0) || (EPI == 2 && again(j1)) ? 1u : 0u) << e;
+          again |= (is(j0) || (EPI == 2 && is(j1)) ? 1u : 0u) << e;
         }
-        redo |= (uint64_t)odd << (4 * (i * TO + j));
-        finish(orow(wave, i), ocol(wave, j), tot[i][j0], tot[i][j1], odd);
+        redo |= (uint64_t)again << (4 * (i * TO + j));
+        finish(orow(wave, i), ocol(wave, j), tot[i][j0], tot[i][j1], again);
       }
-  } else if (active) {
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TO; ++j)
-        finish(orow(wave, i), ocol(wave, j), tot[i][EPI == 2 ? 2 * j : j], tot[i][EPI == 2 ? 2 * j + 1 : j], 0);
   }
   uint64_t* const masks = reinterpret_cast<uint64_t*>(smem);  // (no longer read) by wave and lane
   masks[tid] = redo;
-  if (__ballot(redo != 0) != 0 && lane == 0) any_redo = 1;
   lds_barrier();
-  if (any_redo == 0) return;
 
   // one 16 x 16 block on v_mfma_f32_16x16x4_f32, operands straight from memory
   // (64 columns of K in registers while the 64 before are multiplied)
